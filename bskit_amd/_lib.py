@@ -55,6 +55,12 @@ _SIGS = {
     'bsk_pairs_shell_parts': [_vp, ctypes.POINTER(ctypes.c_ubyte)],
     'bsk_power_spectrum_workspace': [_vp, _c_size_p],
     'bsk_power_spectrum': [_vp, _c_int, _vp, _vp, _vp, _vp],
+    'bsk_blocked_create': [ctypes.POINTER(_vp), _c_int, _c_int, _c_int, _int_p],
+    'bsk_blocked_upload': [_vp],
+    'bsk_blocked_destroy': [_vp],
+    'bsk_blocked_info': [_vp, _c_ll, _c_int, _int_p, _int_p],
+    'bsk_triples_blocked_workspace': [_vp, _c_int, _c_size_p],
+    'bsk_triples_blocked': [_vp, _vp, _vp, _vp, _c_ll, _c_ll, _c_int, _c_double, _vp, _vp, _vp],
     'bsk_triples_plain_workspace': [_c_int, _c_int, _c_size_p],
     'bsk_triples_plain': [_c_int, _vp, _vp, _vp, _c_ll, _c_ll, _c_int, _vp, _c_int, _c_double, _vp,
                           _vp, _vp],

@@ -21,8 +21,9 @@ from . import _lib as L
 # Triple-product paths
 PATH_PLAIN = 'plain'      # one sweep per triangle in the shell precision
 PATH_MFMA = 'mfma'        # split-BF16 MFMA, FP32 accumulate, FP64 reduce
+PATH_BLOCKED = 'blocked'  # the plain path's FP32 sums, one sweep per block of triangles
 PATH_TILED = 'tiled'      # LDS tiled VALU in the shell precision
-PATHS = (PATH_PLAIN, PATH_MFMA, PATH_TILED)
+PATHS = (PATH_PLAIN, PATH_BLOCKED, PATH_MFMA, PATH_TILED)
 
 _MODE = {1: L.MODE_AUTO, 2: L.MODE_AAB, 3: L.MODE_ABC}
 
@@ -227,6 +228,26 @@ class PairPlan:
         try:
             if self.handle:
                 L.lib().bsk_pairs_destroy(self.handle)
+                self.handle = None
+        except Exception:
+            pass
+
+
+class BlockedPlan:
+    """Owner of a bsk_blocked plan: the blocks of triangles of one list."""
+
+    def __init__(self, tri, nshell, mode):
+        tri = np.ascontiguousarray(np.asarray(tri, dtype=np.int32).reshape(-1, 3))
+        h = ctypes.c_void_p()
+        L.call('bsk_blocked_create', ctypes.byref(h), int(mode), int(nshell), len(tri),
+               tri.ctypes.data_as(ctypes.POINTER(ctypes.c_int)))
+        self.handle = h
+        L.call('bsk_blocked_upload', h)
+
+    def __del__(self):
+        try:
+            if self.handle:
+                L.lib().bsk_blocked_destroy(self.handle)
                 self.handle = None
         except Exception:
             pass
@@ -460,6 +481,17 @@ class GridEngine:
             self._tri_cache[key] = r
         return r
 
+    def blocked_plan(self, tri, nshell, mode):
+        """Cached plan of the blocked path for a triangle list."""
+        tri = np.ascontiguousarray(np.asarray(tri, dtype=np.int32).reshape(-1, 3))
+        key = (tri.tobytes(), 'blocked', nshell, mode)
+        r = self._tri_cache.get(key)
+        if r is None:
+            with torch.cuda.device(self.device):
+                r = BlockedPlan(tri, nshell, mode)
+            self._tri_cache[key] = r
+        return r
+
     def mfma_nwg(self, ncell=None):
         """Workgroups of the MFMA kernel: the tuned count, else up to 1024 with
         >= 8 chunks each."""
@@ -612,6 +644,18 @@ class GridEngine:
                        sa.stride, sa.sum_cells, t1 - t0, L.ptr(tri_d[t0:t1]), nchunk, float(scale),
                        L.ptr(out[t0:t1]), L.ptr(w), s)
             return out
+        if path == PATH_BLOCKED:
+            if any(x.fmt != L.FMT_F32 for x in sets):
+                raise ValueError('the blocked path needs F32 shells')
+            nchunk = self.plain_nchunk(ncell)
+            plan = self.blocked_plan(tri, min(x.nb for x in sets), _MODE[nf])
+            nbytes = L.size_out()
+            L.call('bsk_triples_blocked_workspace', plan.handle, nchunk, ctypes.byref(nbytes))
+            w = (work or self.work).get('plain', nbytes.value)
+            L.call('bsk_triples_blocked', plan.handle, L.ptr(sa.data), L.ptr(sb.data),
+                   L.ptr(sc.data), sa.stride, sa.sum_cells, nchunk, float(scale), L.ptr(out),
+                   L.ptr(w), s)
+            return out
         if path == PATH_TILED:
             if nf != 1:
                 raise ValueError('the tiled path takes one shell set (auto spectra)')
@@ -718,7 +762,8 @@ class GridEngine:
                        L.ptr(a.data), L.ptr(a.lo), L.ptr(c.data), L.ptr(c.lo), cells, cells,
                        nwg, float(scale), L.ptr(part), L.ptr(wm), st)
             else:
-                self.triples(sets, tri, path=PATH_PLAIN, scale=scale, out=part, stream=stream)
+                self.triples(sets, tri, path=PATH_PLAIN if f64 else PATH_BLOCKED, scale=scale,
+                             out=part, stream=stream)
             with torch.cuda.stream(stream if stream is not None else
                                    torch.cuda.current_stream(self.device)):
                 out += part

@@ -317,7 +317,7 @@ class FFTBispectrum:
                                dtype=torch.float32 if fmt != L.FMT_F64 else torch.float64)
                 self._shells[skey] = s
             sets.append(s)
-        path = 'mfma' if fmt == L.FMT_BF16X2 else 'plain'
+        path = {L.FMT_BF16X2: 'mfma', L.FMT_F32: 'blocked', L.FMT_F64: 'plain'}[fmt]
         return sets, path
 
     def _unnorm_sums(self, kLU, tri, factor):

@@ -210,6 +210,30 @@ int bsk_triples_plain(int dtype, const void* fa, const void* fb, const void* fc,
                       long long shell_stride, long long ncell, int ntri, const int* tri_dev,
                       int nchunk, double scale, double* out_dev, void* work, void* stream);
 
+/* The FP32 sums of bsk_triples_plain over blocks of triangles: out[t] =
+ * scale * sum_x A[i_t](x) B[j_t](x) C[k_t](x), one sweep over the cells per
+ * block of up to 4 x 4 x 4 triangles instead of one per triangle.  At the same
+ * nchunk the sums are the same bits as bsk_triples_plain's.  A plan (host
+ * tables, uploaded once) groups the list's triangles; mode as in
+ * bsk_pairs_create (BSK_MODE_ABC: sides i and j come from different sets and
+ * are not exchanged), shell indices below nshell.  Replaces the per-triangle
+ * loop of measure_bispectrum_faster (bskit/main.py:1871-1882).  Cell count
+ * and shell stride are multiples of 4.
+ * work: bsk_triples_blocked_workspace() bytes. */
+typedef struct bsk_blocked bsk_blocked;
+int bsk_blocked_create(bsk_blocked** plan, int mode, int nshell, int ntri, const int* tri_host);
+int bsk_blocked_upload(bsk_blocked* plan);
+int bsk_blocked_destroy(bsk_blocked* plan);
+/* Distinct triangles of the list, and the kernel a call with ncell cells and
+ * nchunk chunks runs (0: one sweep per triangle, 1: blocks of 2 x 2 x 2, 2: of
+ * 4 x 4 x 4). */
+int bsk_blocked_info(const bsk_blocked* plan, long long ncell, int nchunk, int* nrow,
+                     int* kernel);
+int bsk_triples_blocked_workspace(const bsk_blocked* plan, int nchunk, size_t* bytes);
+int bsk_triples_blocked(const bsk_blocked* plan, const float* fa, const float* fb,
+                        const float* fc, long long shell_stride, long long ncell, int nchunk,
+                        double scale, double* out_dev, void* work, void* stream);
+
 /* LDS-tiled triple sums over fields[0..nfield) (stride shell_stride).
  * nsum = 1: out[t] = scale * sum_x F[i] F[j] F[k].
  * nsum = 4: fields are nfield/2 unit shells then nfield/2 |k| shells and
