@@ -774,6 +774,7 @@ constexpr unsigned kPartLevels[kParts] = {0x3, 0xf, 0x5, 0x1};
 static_assert(kParts == kPairSlots, "one partial slot per triangle and segment");
 
 struct bsk_pairs {
+  bool f64 = false;    // for the FP64 kernel (dpairs.hip), else the split-BF16 one
   int mode = 0;
   int nshell = 0;
   int sets = 1;
@@ -856,7 +857,11 @@ PairTiles build_tiles(const std::vector<Role>& roles, bool exact) {
 // (VALU) and reads both pair sides from LDS; an item reads one third-side
 // block and issues three MFMAs.  Measured on gfx950 a tile costs about
 // three items.
-int plan_cost(const PairTiles& t) { return 3 * (int)t.tile_mask.size() + t.nitem; }
+// In FP64 an item is 128 cycles of MFMA per eight cells and a tile two
+// multiplies a lane: the items decide.
+int plan_cost(const PairTiles& t, bool f64) {
+  return f64 ? (int)t.tile_mask.size() + 8 * t.nitem : 3 * (int)t.tile_mask.size() + t.nitem;
+}
 
 std::vector<Role> assign_roles(int mode, int option, int ntri, const int* tri) {
   std::vector<Role> r(ntri);
@@ -965,7 +970,8 @@ struct LevelPlan {
   int lo = 0, hi = 0;  // shells used: [lo, hi)
 };
 
-LevelPlan plan_level(int mode, int nkb, int cap, const std::vector<int>& idx, const int* tri) {
+LevelPlan plan_level(int mode, int nkb, int cap, const std::vector<int>& idx, const int* tri,
+                     bool f64) {
   LevelPlan lp;
   lp.tri = idx;
   std::vector<int> sub((size_t)3 * idx.size());
@@ -987,7 +993,7 @@ LevelPlan plan_level(int mode, int nkb, int cap, const std::vector<int>& idx, co
         o == 3 ? assign_roles_cover(ntri, sub.data()) : assign_roles(mode, o, ntri, sub.data());
     for (int exact = 1; exact >= 0; --exact) {
       PairTiles t = build_tiles(r, exact != 0);
-      if (first || plan_cost(t) < plan_cost(lp.tiles)) {
+      if (first || plan_cost(t, f64) < plan_cost(lp.tiles, f64)) {
         lp.roles = r;
         lp.tiles = t;
         first = false;
@@ -1017,17 +1023,17 @@ LevelPlan plan_level(int mode, int nkb, int cap, const std::vector<int>& idx, co
 }
 
 // Units (tile, kb mask) to (pass, wave) bins, costliest first (forming a
-// tile's products weighs three items), each to the cheapest bin with room for
+// tile's products weighs `form` items), each to the cheapest bin with room for
 // its items; the fewest passes for which every unit fits.
 std::vector<std::vector<int>> bin_units(const std::vector<unsigned>& mask, int cap, int W,
-                                        int* npass, int* maxload) {
+                                        int* npass, int* maxload, int form = 3) {
   const int nunit = (int)mask.size();
   int nitem = 0;
   for (unsigned m : mask) {
     nitem += __builtin_popcount(m);
     cap = std::max(cap, __builtin_popcount(m));  // every unit fits an empty bin
   }
-  auto ucost = [&](int u) { return 3 + __builtin_popcount(mask[u]); };
+  auto ucost = [&](int u) { return form + __builtin_popcount(mask[u]); };
   std::vector<int> order(nunit);
   for (int i = 0; i < nunit; ++i) order[i] = i;
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return ucost(x) > ucost(y); });
@@ -1061,7 +1067,7 @@ std::vector<std::vector<int>> bin_units(const std::vector<unsigned>& mask, int c
 }
 
 int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri,
-                 const int* level, const char* fn) {
+                 const int* level, const char* fn, bool f64 = false) {
   if (!out || nshell < 1 || mode < 0 || mode > 2 || ntri < 0 || (ntri && !tri)) {
     bsk_set_error("%s: invalid argument", fn);
     return BSK_EINVAL;
@@ -1081,8 +1087,13 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
   const int sets = mode == BSK_MODE_AUTO ? 1 : (mode == BSK_MODE_AAB ? 2 : 3);
   const int nkb = (nshell + 15) / 16;
   int nsh[3] = {nshell, nshell, nshell};
-  if (!bsk_pair_prefetch(nshell) || bsk_pair_lds_bytes(sets, nsh, nkb + 1) > 160 * 1024 ||
-      nkb > 16 || nshell >= 0xffff) {
+  if (f64) {
+    if (!bsk_dpair_fits(sets, nshell)) {
+      bsk_set_error("%s: %d shells exceed the FP64 kernel's staging", fn, nshell);
+      return BSK_EUNSUPPORTED;
+    }
+  } else if (!bsk_pair_prefetch(nshell) || bsk_pair_lds_bytes(sets, nsh, nkb + 1) > 160 * 1024 ||
+             nkb > 16 || nshell >= 0xffff) {
     bsk_set_error("%s: %d shells exceed the MFMA kernel's LDS staging "
                   "(128 shells, 96 for <ABC>)", fn, nshell);
     return BSK_EUNSUPPORTED;
@@ -1090,7 +1101,8 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
   // at most 4 items per wave per launch keeps two workgroups per CU (more
   // items of a segment take more launches over its cells); units (a tile's
   // items formed from one set of pair products) hold at most that many
-  const int W = kPairWaves, cap = std::min(4, bsk_pair_item_cap(sets, nshell));
+  const int W = kPairWaves,
+            cap = f64 ? kDPairMaxItems : std::min(4, bsk_pair_item_cap(sets, nshell));
   std::vector<int> idx[BSK_LEVELS];
   for (int t = 0; t < ntri; ++t) idx[level ? level[t] : 0].push_back(t);
   unsigned present = 0;
@@ -1125,7 +1137,7 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
     for (int L = 0; L < BSK_LEVELS; ++L)
       if (segs[g].lv >> L & 1) sel.insert(sel.end(), idx[L].begin(), idx[L].end());
     std::sort(sel.begin(), sel.end());
-    lp[g] = plan_level(mode, nkb, cap, sel, tri);
+    lp[g] = plan_level(mode, nkb, cap, sel, tri, f64);
     tile0[g + 1] = tile0[g] + (int)lp[g].tiles.tile_mask.size();
   }
   const int ntile = tile0[nseg];
@@ -1167,6 +1179,22 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
     if (sp[g].unit_mask.empty()) {
       sp[g].npass = 1;
       sp[g].bins.assign(W, {});
+    } else if (f64) {
+      // lists on W / rep waves, replicated rep times, each replica running
+      // every rep-th K step: the count that leaves the fullest wave the least
+      double best = 0.0;
+      for (int rep : {1, 2, 4, 8}) {
+        int np = 0, m2 = 1;
+        auto b2 = bin_units(sp[g].unit_mask, cap, W / rep, &np, &m2, 0);
+        const double t = (double)np * bsk_dpair_items_round(m2) / rep;
+        if (rep > 1 && (np > 1 || t >= best)) continue;
+        best = t;
+        ml = m2;
+        sp[g].npass = np;
+        sp[g].rep = rep;
+        sp[g].bins.clear();
+        for (int r = 0; r < rep; ++r) sp[g].bins.insert(sp[g].bins.end(), b2.begin(), b2.end());
+      }
     } else {
       sp[g].bins = bin_units(sp[g].unit_mask, cap, W, &sp[g].npass, &ml);
       // few items (a plan over levels): lists on W / rep waves, replicated
@@ -1197,7 +1225,7 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
         }
       }
     }
-    sp[g].ni = bsk_pair_items_round(ml);
+    sp[g].ni = f64 ? bsk_dpair_items_round(ml) : bsk_pair_items_round(ml);
     maxni = std::max(maxni, sp[g].ni);
     nentry += (size_t)sp[g].npass * W * sp[g].ni;
   }
@@ -1273,6 +1301,7 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
     }
     npair += (int)tl.pairs.size();
   }
+  q->f64 = f64;
   q->mode = mode;
   q->nshell = nshell;
   q->sets = sets;
@@ -1417,6 +1446,11 @@ int bsk_triples_mfma_workspace(const bsk_pairs* q, int nwg, size_t* bytes) {
     bsk_set_error("bsk_triples_mfma_workspace: invalid argument");
     return BSK_EINVAL;
   }
+  if (q->f64) {
+    *bytes = sizeof(double) * 256 * (size_t)q->item_total * nwg +
+             bsk_reduce_dpairs_bytes(q->item_total);
+    return BSK_OK;
+  }
   // per-workgroup FP32 partials, then the reduction's FP64 range sums
   *bytes = sizeof(float) * 256 * (size_t)q->item_total * nwg + bsk_reduce_mfma_bytes(q->item_total);
   return BSK_OK;
@@ -1430,6 +1464,39 @@ double* reduce_scratch(void* work, const bsk_pairs* q, int nwg) {
 }  // namespace
 
 namespace {
+// Cell range [beg, end) of each layout part in a shell row: P1 = level 3, P0 =
+// the rest of level 1 before it, P2 = the rest of level 2 after it, P3 = the
+// rest of level 0; the whole row for C order (no level ranges).
+int part_ranges(const bsk_pairs* q, long long shell_stride, long long ncell,
+                const long long* level_off, const long long* level_ncell, int chunk,
+                long long (&pbeg)[kParts], long long (&pend)[kParts], const char* fn,
+                const char* levels_fn) {
+  if (level_off && level_ncell) {
+    const long long* o = level_off;
+    const long long* n = level_ncell;
+    pbeg[0] = o[1], pend[0] = o[3];
+    pbeg[1] = o[3], pend[1] = o[3] + n[3];
+    pbeg[2] = o[3] + n[3], pend[2] = o[2] + n[2];
+    pbeg[3] = o[2] + n[2], pend[3] = o[0] + n[0];
+    bool ok = o[0] == o[1] && o[2] == o[3] && o[0] <= o[3] && o[0] + n[0] <= shell_stride;
+    for (int p = 0; p < kParts; ++p)
+      ok = ok && pbeg[p] <= pend[p] && pbeg[p] % chunk == 0 && pend[p] % chunk == 0;
+    if (!ok) {
+      bsk_set_error("%s: level ranges do not nest as the level layout's (bsk_plan_levels)", fn);
+      return BSK_EINVAL;
+    }
+    return BSK_OK;
+  }
+  if (q->nseg != 1 || q->seg_parts[0] != 0xf) {
+    bsk_set_error("%s: the plan has sublattice-level triangles; use %s with the bsk_plan_levels "
+                  "layout", fn, levels_fn);
+    return BSK_EINVAL;
+  }
+  std::fill(pbeg, pbeg + kParts, 0LL);
+  std::fill(pend, pend + kParts, ncell);
+  return BSK_OK;
+}
+
 int triples_mfma(const bsk_pairs* q, const uint16_t* hi_i, const uint16_t* lo_i,
                  const uint16_t* hi_j, const uint16_t* lo_j, const uint16_t* hi_k,
                  const uint16_t* lo_k, long long shell_stride, long long ncell,
@@ -1440,33 +1507,14 @@ int triples_mfma(const bsk_pairs* q, const uint16_t* hi_i, const uint16_t* lo_i,
     bsk_set_error("%s: invalid argument", fn);
     return BSK_EINVAL;
   }
-  // cell range of each layout part: P1 = level 3, P0 = the rest of level 1
-  // before it, P2 = the rest of level 2 after it, P3 = the rest of level 0
-  long long pbeg[kParts], pend[kParts];
-  if (level_off && level_ncell) {
-    const long long* o = level_off;
-    const long long* n = level_ncell;
-    pbeg[0] = o[1], pend[0] = o[3];
-    pbeg[1] = o[3], pend[1] = o[3] + n[3];
-    pbeg[2] = o[3] + n[3], pend[2] = o[2] + n[2];
-    pbeg[3] = o[2] + n[2], pend[3] = o[0] + n[0];
-    bool ok = o[0] == o[1] && o[2] == o[3] && o[0] <= o[3] && o[0] + n[0] <= shell_stride;
-    for (int p = 0; p < kParts; ++p)
-      ok = ok && pbeg[p] <= pend[p] && pbeg[p] % kPairChunk == 0 && pend[p] % kPairChunk == 0;
-    if (!ok) {
-      bsk_set_error("%s: level ranges do not nest as the level layout's (bsk_plan_levels)", fn);
-      return BSK_EINVAL;
-    }
-  } else {
-    if (q->nseg != 1 || q->seg_parts[0] != 0xf) {
-      bsk_set_error("%s: the plan has sublattice-level triangles; use bsk_triples_mfma_levels "
-                    "with the bsk_plan_levels layout", fn);
-      return BSK_EINVAL;
-    }
-    // one segment of all parts: the whole C-order range
-    std::fill(pbeg, pbeg + kParts, 0LL);
-    std::fill(pend, pend + kParts, ncell);
+  if (q->f64) {
+    bsk_set_error("%s: the plan is for the FP64 sums (bsk_triples_f64)", fn);
+    return BSK_EINVAL;
   }
+  long long pbeg[kParts], pend[kParts];
+  if (int rc = part_ranges(q, shell_stride, ncell, level_off, level_ncell, kPairChunk, pbeg, pend,
+                           fn, "bsk_triples_mfma_levels"))
+    return rc;
   if (q->ntri == 0) return BSK_OK;
   if (!q->d_items) {
     bsk_set_error("%s: pair plan not uploaded (bsk_pairs_upload)", fn);
@@ -1607,6 +1655,7 @@ namespace {
 // Why the fused z/triple kernel cannot run this plan (nullptr: it can).
 const char* zfused_gap(const bsk_plan* p, const bsk_pairs* q) {
   if (!p || !q) return "null plan";
+  if (q->f64) return "the plan is for the FP64 sums";
   if (q->mode != BSK_MODE_AUTO) return "auto spectra only";
   if (q->nseg != 1 || q->seg_parts[0] != 0xf) return "the plan has sublattice-level triangles";
   const int nsh = q->seg_win[0][1];  // shells staged: the plan's window
@@ -1687,13 +1736,79 @@ int bsk_triples_zfused(bsk_plan* p, const bsk_pairs* q, const void* shell_work, 
 
 int bsk_triples_mfma_reduce(const bsk_pairs* q, int nwg, double scale, double* out_dev,
                             void* work, void* stream) {
-  if (!q || nwg <= 0 || !out_dev || !work || !q->d_slot) {
+  if (!q || q->f64 || nwg <= 0 || !out_dev || !work || !q->d_slot) {
     bsk_set_error("bsk_triples_mfma_reduce: invalid argument (plan uploaded?)");
     return BSK_EINVAL;
   }
   return bsk_reduce_mfma_launch(reinterpret_cast<const float*>(work), nwg, q->item_total,
                                 q->ntri, q->d_slot, scale, out_dev, reduce_scratch(work, q, nwg),
                                 as_stream(stream));
+}
+
+// ------------------------------------------------------------------ FP64
+int bsk_pairs_create_f64(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri,
+                         const int* level) {
+  return pairs_create(out, mode, nshell, ntri, tri, level, "bsk_pairs_create_f64", true);
+}
+
+int bsk_triples_f64(const bsk_pairs* q, const double* f_i, const double* f_j, const double* f_k,
+                    long long shell_stride, long long ncell, const long long* level_off,
+                    const long long* level_ncell, const double* weight, int nwg, double scale,
+                    double* out_dev, void* work, void* stream) {
+  const char* fn = "bsk_triples_f64";
+  if (!q || !f_j || !out_dev || !work || nwg <= 0 || shell_stride < ncell ||
+      (q->mode >= 1 && !f_k) || (q->mode == 2 && !f_i) || (level_off == nullptr) != (level_ncell == nullptr)) {
+    bsk_set_error("%s: invalid argument", fn);
+    return BSK_EINVAL;
+  }
+  if (!q->f64) {
+    bsk_set_error("%s: the plan is for the split-BF16 sums (bsk_pairs_create_f64)", fn);
+    return BSK_EINVAL;
+  }
+  long long pbeg[kParts], pend[kParts];
+  if (int rc = part_ranges(q, shell_stride, ncell, level_off, level_ncell, kDPairChunk, pbeg, pend,
+                           fn, "level ranges"))
+    return rc;
+  if (q->ntri == 0) return BSK_OK;
+  if (!q->d_items) {
+    bsk_set_error("%s: pair plan not uploaded (bsk_pairs_upload)", fn);
+    return BSK_EINVAL;
+  }
+  DPairArgs a = {};
+  const double* f[3] = {q->mode == 2 ? f_i : f_j, f_j, q->mode >= 1 ? f_k : f_j};
+  a.stride = shell_stride;
+  a.nwg = nwg;
+  a.pairs = q->d_pairs;
+  a.partial = reinterpret_cast<double*>(work);
+  a.item_total = q->item_total;
+  hipStream_t s = as_stream(stream);
+  size_t e0 = 0;  // first list entry of the launch
+  for (int g = 0; g < q->nseg; ++g) {  // as triples_mfma's
+    const int fp = __builtin_ctz(q->seg_parts[g]), lp = 31 - __builtin_clz(q->seg_parts[g]);
+    const int w0 = q->seg_win[g][0], wn = q->seg_win[g][1];
+    const long long base = pbeg[fp] + (long long)w0 * shell_stride;
+    for (int r = 0; r < 3; ++r) a.f[r] = f[r] + base;
+    a.weight = weight ? weight + pbeg[fp] : nullptr;
+    a.nsh = wn;
+    a.lo_row = w0;
+    a.koff = w0 % 16;
+    a.nkb = (a.koff + wn + 15) / 16;
+    a.ncell = pend[lp] - pbeg[fp];
+    a.rep = q->seg_rep[g];
+    const int ni = q->seg_ni[g], np = q->seg_pass[g];
+    const bool fold = np > 1 && nwg % 8 == 0;
+    a.npass = fold ? np : 1;
+    a.pass_stride = kPairWaves * ni;
+    for (int k = 0; k < np; k += a.npass) {
+      a.items = q->d_items + e0 + (size_t)k * kPairWaves * ni;
+      a.outpos = q->d_outpos + e0 + (size_t)k * kPairWaves * ni;
+      if (int rc = bsk_triple_dpairs_launch(a, q->sets, ni, s)) return rc;
+    }
+    e0 += (size_t)np * kPairWaves * ni;
+  }
+  double* sums = a.partial + (size_t)256 * q->item_total * nwg;
+  return bsk_reduce_dpairs_launch(a.partial, nwg, q->item_total, q->ntri, q->d_slot, scale, out_dev,
+                                  sums, s);
 }
 
 }  // extern "C"

@@ -1,0 +1,293 @@
+// FP64 MFMA triple sums over a list of shell pairs:
+//   B[i][j][k] = sum_x w(x) (d_i d_j)(x) d_k(x)   (w = 1 without weights).
+//
+// The pair plan is mfma.hip's (tiles of 16 pairs, items of a tile and a block
+// of 16 third-side shells, launch segments over the sublattice levels), the
+// arithmetic all FP64: a K step of eight cells is, per item, two
+// v_mfma_f64_16x16x4 on the pair products (A) and the shells (B).  One item
+// costs 512 multiply-adds per cell whatever its tile needs of them, but its
+// 16 x 16 accumulators are 8 VGPRs a lane, so eight waves hold every item of
+// a segment and the shells are read once; a register-blocked sum of single
+// triangles (blocked.hip's scheme in FP64) holds 64 triangles a wave and read
+// the shells 13 times: 5.0 ms at 512^3 / 32 bins, one sweep per triangle 84 ms,
+// this 0.74 ms over the levels (2.1 without them).  FP64 MFMA and FP64 VALU
+// have the same peak on gfx950 (72 TFLOP/s measured with a large matrix
+// product) and share issue time, so what bounds it is the MFMAs (0.52 ms of
+// the 0.74 at 2.17 GHz) plus every VALU instruction between them: the K loop
+// is rolled with one address add per LDS read.
+//
+// Workgroup: eight waves over a contiguous range of 64-cell chunks; per chunk
+// the staged shells' rows go from HBM through registers (loaded one chunk
+// ahead) into LDS, FP64 rows of 68 (544 B: the row stride that serves 16-B
+// reads of 16 arbitrary rows best).  Lane (col, grp) of a wave reads cells 2
+// grp and 2 grp + 1 of an eight-cell K step, of its pair's two rows and of its
+// third-side row; the first MFMA takes the even cells, the second the odd
+// ones.  A segment with few items replicates its wave lists over 2, 4 or 8
+// wave groups that take alternate K steps.
+#include <algorithm>
+
+#include "launch.h"
+
+namespace {
+
+constexpr int kW = kPairWaves;
+constexpr int kNT = 64 * kW;
+constexpr int kCK = kDPairChunk;      // cells per staged chunk
+constexpr int kLD = kCK + 4;          // LDS row stride (doubles)
+constexpr int kSEG = kCK / 2;         // 16-byte segments per row
+constexpr int kSteps = kCK / 8;       // K steps of eight cells per chunk
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));
+
+// Rows of LDS before each set's: set 0 (pair sides, and the third side of an
+// auto spectrum), set 1 (<ABC>), set 2 (third side), the weights.
+struct Rows {
+  int r1, r2, rw;
+};
+__host__ __device__ inline Rows lds_rows(int sets, int n0, int n1, int nkb) {
+  Rows r;
+  r.r1 = sets == 1 ? 16 * nkb : n0;
+  r.r2 = sets == 1 ? 0 : (sets == 3 ? n0 + n1 : n0);
+  r.rw = sets == 1 ? 16 * nkb : r.r2 + 16 * nkb;
+  return r;
+}
+
+template <int NI, int PV, int SETS, bool WT>
+__global__ __launch_bounds__(kNT, 2) void k_triple_dpairs(DPairArgs a) {
+  extern __shared__ __attribute__((aligned(16))) double smem[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rep = a.rep, rgrp = wave / (kW / rep);
+  const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+  const Rows R = lds_rows(SETS, a.nsh, a.nsh, a.nkb);
+  // LDS row of staged shell 0 of each set: the third side's blocks are
+  // 16-aligned, so it starts at koff
+  const int s0 = SETS == 1 ? a.koff : 0, s1 = R.r1, s2 = R.r2 + a.koff;
+
+  int lw = blockIdx.x, pass = 0;  // cell range and item-list pass (see PairArgs)
+  if (a.npass > 1) {
+    pass = (blockIdx.x >> 3) % a.npass;
+    lw = (blockIdx.x / (8 * a.npass)) * 8 + (blockIdx.x & 7);
+  }
+  const int* items = a.items + pass * a.pass_stride + wave * NI;
+  const int* outpos = a.outpos + pass * a.pass_stride + wave * NI;
+  // per item: descriptor, this lane's offsets of its pair rows (padding rows
+  // read row 0: their sums are never read) and of its third-side row
+  int desc[NI], oi[NI], oj[NI], ok[NI];
+#pragma unroll
+  for (int s = 0; s < NI; ++s) {
+    desc[s] = __builtin_amdgcn_readfirstlane(items[s]);
+    const int pr = a.pairs[(desc[s] & 0xffff) * 16 + col];
+    const int ra = pr & 0xffff, rb = (pr >> 16) & 0xffff;
+    const int ia = ra == 0xffff ? 0 : ra - a.lo_row, ib = rb == 0xffff ? 0 : rb - a.lo_row;
+    oi[s] = (s0 + ia) * kLD + 2 * grp;
+    oj[s] = ((SETS == 3 ? s1 : s0) + ib) * kLD + 2 * grp;
+    ok[s] = (R.r2 + 16 * ((desc[s] >> 16) & 0xff) + col) * kLD + 2 * grp;
+  }
+  d4 acc[NI];
+#pragma unroll
+  for (int s = 0; s < NI; ++s) acc[s] = d4{0.0, 0.0, 0.0, 0.0};
+
+  // staging: segment v = thread + k kNT is 16 bytes of staged row v / kSEG:
+  // the shells of set 0, then 1, then 2, then the weights
+  const int n = a.nsh, nrow = SETS * n + (WT ? 1 : 0);
+  const long long nch = a.ncell / kCK;
+  const long long ch0 = nch * lw / a.nwg, ch1 = nch * (lw + 1) / a.nwg;
+  const double* src[PV];
+  int dst[PV];
+#pragma unroll
+  for (int k = 0; k < PV; ++k) {
+    const int v = threadIdx.x + k * kNT, row = v / kSEG, sg = v % kSEG;
+    const int set = row < n ? 0 : (row < 2 * n ? 1 : 2);  // the set's place in the list
+    const int sh = row - set * n;
+    const bool wt = WT && row == nrow - 1;
+    const double* base = set == 0 ? a.f[0] : (SETS == 3 && set == 1 ? a.f[1] : a.f[2]);
+    const int lrow = set == 0 ? s0 : (SETS == 3 && set == 1 ? s1 : s2);
+    src[k] = wt ? a.weight + 2 * sg + ch0 * kCK : base + sh * a.stride + 2 * sg + ch0 * kCK;
+    dst[k] = row < nrow ? (wt ? R.rw : lrow + sh) * kLD + 2 * sg : -1;
+  }
+  d2 pre[PV];
+  auto fetch = [&]() {
+#pragma unroll
+    for (int k = 0; k < PV; ++k) {
+      if (dst[k] >= 0) pre[k] = *reinterpret_cast<const d2*>(src[k]);
+      src[k] += kCK;
+    }
+  };
+  if (ch0 < ch1) fetch();
+  for (long long ch = ch0; ch < ch1; ++ch) {
+    __syncthreads();  // every wave is done with the previous chunk
+#pragma unroll
+    for (int k = 0; k < PV; ++k)
+      if (dst[k] >= 0) *reinterpret_cast<d2*>(smem + dst[k]) = pre[k];
+    __syncthreads();
+    if (ch + 1 < ch1) fetch();  // the next chunk's loads overlap this one's math
+    for (int ks = rgrp; ks < kSteps; ks += rep) {
+      int o = 8 * ks;
+      asm("" : "+s"(o));  // keeps one add per read, not an induction variable per row
+      const double* f = smem + o;
+      d2 p = {0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < NI; ++s) {
+        if (desc[s] & (1 << 29)) continue;  // uniform: padding item
+        const d2 z = *reinterpret_cast<const d2*>(f + ok[s]);
+        if (s == 0 || desc[s] < 0) {        // uniform: new tile, new pair products
+          const d2 x = *reinterpret_cast<const d2*>(f + oi[s]);
+          const d2 y = *reinterpret_cast<const d2*>(f + oj[s]);
+          p = {x.x * y.x, x.y * y.y};
+          if (WT) {
+            const d2 w = *reinterpret_cast<const d2*>(f + R.rw * kLD + 2 * grp);
+            p = {p.x * w.x, p.y * w.y};
+          }
+        }
+        acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(p.x, z.x, acc[s], 0, 0, 0);
+        acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(p.y, z.y, acc[s], 0, 0, 0);
+      }
+    }
+  }
+  // replicas of a wave's list ran other K steps: the first adds theirs
+  // through LDS and stores
+  if (rep > 1) {
+    const int wpr = kW / rep, wl = wave % wpr;
+    for (int g = 1; g < rep; ++g) {
+      __syncthreads();
+      if (rgrp == g)
+#pragma unroll
+        for (int s = 0; s < NI; ++s)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) smem[((wl * NI + s) * 4 + r) * 64 + lane] = acc[s][r];
+      __syncthreads();
+      if (rgrp == 0)
+#pragma unroll
+        for (int s = 0; s < NI; ++s)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[s][r] += smem[((wl * NI + s) * 4 + r) * 64 + lane];
+    }
+    if (rgrp) return;
+  }
+  // C[row][col]: register r of lane group grp is row 4 r + grp
+  double* const out = a.partial + (long long)lw * a.item_total * 256;
+#pragma unroll
+  for (int s = 0; s < NI; ++s) {
+    const int pos = __builtin_amdgcn_readfirstlane(outpos[s]);
+    if (pos < 0) continue;  // uniform
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out[(long long)pos * 256 + (4 * r + grp) * 16 + col] = acc[s][r];
+  }
+}
+
+template <int NI, int PV, int SETS>
+int launch(const DPairArgs& a, size_t lds, hipStream_t s) {
+  auto go = [&](auto fn, hipError_t attr) {
+    BSK_HIP_CHECK(attr);
+    hipLaunchKernelGGL(fn, dim3(a.nwg * a.npass), dim3(kNT), lds, s, a);
+    BSK_LAUNCH_CHECK();
+    return BSK_OK;
+  };
+  constexpr int kMax = 160 * 1024;
+  if constexpr (SETS == 1) {
+    if (a.weight) {
+      static const hipError_t attr =
+          hipFuncSetAttribute((const void*)k_triple_dpairs<NI, PV, SETS, true>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, kMax);
+      return go(k_triple_dpairs<NI, PV, SETS, true>, attr);
+    }
+  }
+  static const hipError_t attr =
+      hipFuncSetAttribute((const void*)k_triple_dpairs<NI, PV, SETS, false>,
+                          hipFuncAttributeMaxDynamicSharedMemorySize, kMax);
+  return go(k_triple_dpairs<NI, PV, SETS, false>, attr);
+}
+
+template <int PV, int SETS>
+int launch_ni(const DPairArgs& a, int ni, size_t lds, hipStream_t s) {
+  switch (ni) {
+    case 1: return launch<1, PV, SETS>(a, lds, s);
+    case 2: return launch<2, PV, SETS>(a, lds, s);
+    case 3: return launch<3, PV, SETS>(a, lds, s);
+    case 4: return launch<4, PV, SETS>(a, lds, s);
+    case 6: return launch<6, PV, SETS>(a, lds, s);
+    case 8: return launch<8, PV, SETS>(a, lds, s);
+  }
+  bsk_set_error("FP64 pair sums: %d items per wave not compiled", ni);
+  return BSK_EUNSUPPORTED;
+}
+
+template <int SETS>
+int launch_pv(const DPairArgs& a, int ni, int pv, size_t lds, hipStream_t s) {
+  if (pv <= 3) return launch_ni<3, SETS>(a, ni, lds, s);
+  if (pv <= 5) return launch_ni<5, SETS>(a, ni, lds, s);
+  if (pv <= 10) return launch_ni<10, SETS>(a, ni, lds, s);
+  if (pv <= 18) return launch_ni<18, SETS>(a, ni, lds, s);
+  bsk_set_error("FP64 pair sums: %d prefetch segments per thread not compiled", pv);
+  return BSK_EUNSUPPORTED;
+}
+
+// FP64 partials summed over the workgroups of each of kRedSplit ranges.
+__global__ __launch_bounds__(256) void k_reduce_dslots(const double* __restrict__ partial, int nwg,
+                                                       int nslot, double* __restrict__ sums) {
+  const int e = blockIdx.x * 256 + threadIdx.x, c = blockIdx.y;
+  if (e >= nslot) return;
+  const int w0 = (int)((long long)nwg * c / kRedSplit), w1 = (int)((long long)nwg * (c + 1) / kRedSplit);
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  int w = w0;
+  for (; w + 4 <= w1; w += 4)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s[k] += partial[(long long)(w + k) * nslot + e];
+  for (; w < w1; ++w) s[0] += partial[(long long)w * nslot + e];
+  sums[(long long)c * nslot + e] = (s[0] + s[1]) + (s[2] + s[3]);
+}
+
+}  // namespace
+
+int bsk_dpair_items_round(int ni) { return ni <= 4 ? std::max(ni, 1) : (ni <= 6 ? 6 : (ni <= 8 ? 8 : 0)); }
+
+bool bsk_dpair_fits(int sets, int nshell) {
+  const int nkb = (nshell + 15) / 16 + 1;  // a window may start inside a block
+  const int rows = lds_rows(sets, nshell, nshell, nkb).rw + 1;
+  return sets * nshell + 1 <= 18 * kNT / kSEG && (size_t)rows * kLD * 8 <= 160 * 1024;
+}
+
+int bsk_triple_dpairs_launch(const DPairArgs& a, int sets, int ni, hipStream_t s) {
+  if (a.ncell % kCK || a.stride % 2 || a.nwg <= 0 || a.nsh < 1) {
+    bsk_set_error("FP64 pair sums: cells in multiples of %d, even stride, nwg > 0", kCK);
+    return BSK_EINVAL;
+  }
+  if (a.npass < 1 || (a.npass > 1 && (a.nwg % 8 || a.rep != 1))) {
+    bsk_set_error("FP64 pair sums: folded passes need nwg a multiple of 8 and no replicas");
+    return BSK_EINVAL;
+  }
+  if (a.rep != 1 && a.rep != 2 && a.rep != 4 && a.rep != 8) {
+    bsk_set_error("FP64 pair sums: %d replicas (1, 2, 4 or 8)", a.rep);
+    return BSK_EINVAL;
+  }
+  const size_t rows = (size_t)lds_rows(sets, a.nsh, a.nsh, a.nkb).rw + (a.weight ? 1 : 0);
+  const size_t lds = std::max(rows * kLD * 8, a.rep > 1 ? (size_t)(kW / a.rep) * ni * 256 * 8 : 0);
+  const int pv = ((sets * a.nsh + (a.weight ? 1 : 0)) * kSEG + kNT - 1) / kNT;
+  if (lds > 160 * 1024) {
+    bsk_set_error("FP64 pair sums: %d shells exceed the kernel's staging", a.nsh);
+    return BSK_EUNSUPPORTED;
+  }
+  if (sets == 1) return launch_pv<1>(a, ni, pv, lds, s);
+  if (a.weight) {
+    bsk_set_error("FP64 pair sums: weights with one shell set only");
+    return BSK_EINVAL;
+  }
+  if (sets == 2) return launch_pv<2>(a, ni, pv, lds, s);
+  return launch_pv<3>(a, ni, pv, lds, s);
+}
+
+size_t bsk_reduce_dpairs_bytes(int items_per_wg) {
+  return sizeof(double) * kRedSplit * 256 * (size_t)items_per_wg;
+}
+
+int bsk_reduce_dpairs_launch(const double* partial, int nwg, int items_per_wg, int ntri,
+                             const int* slot, double scale, double* out, double* sums,
+                             hipStream_t s) {
+  if (ntri <= 0) return BSK_OK;
+  const int nslot = items_per_wg * 256;
+  hipLaunchKernelGGL(k_reduce_dslots, dim3((nslot + 255) / 256, kRedSplit), dim3(256), 0, s, partial,
+                     nwg, nslot, sums);
+  BSK_LAUNCH_CHECK();
+  return bsk_reduce_tri_launch(sums, nslot, ntri, slot, scale, out, s);
+}

@@ -104,6 +104,39 @@ int bsk_reduce_mfma_launch(const float* partial, int nwg, int items_per_wg, int 
                            const int* slot_dev, double scale, double* out, double* sums,
                            hipStream_t s);
 
+// FP64 MFMA path over pair lists (dpairs.hip); the plan's tables as PairArgs'.
+constexpr int kDPairChunk = 64;   // cells per staged chunk
+constexpr int kDPairMaxItems = 8; // items per wave and launch
+struct DPairArgs {
+  const double* f[3];     // role sets: first pair side, second, third side
+  long long stride;       // elements between consecutive shells of a set
+  int nsh;                // shells staged per role set
+  int nkb;                // 16-shell blocks of the third side staged in LDS
+  int lo_row, koff;       // shell of staged row 0; its third-side LDS row
+  long long ncell;        // cells per shell (multiple of kDPairChunk)
+  int nwg;
+  const int* items;
+  const int* outpos;
+  int rep;                // replicas of the wave lists (1, 2, 4, 8)
+  const int* pairs;
+  double* partial;        // [nwg][item_total][256]
+  int item_total;
+  int npass, pass_stride;
+  const double* weight;   // per cell, or null (one shell set only)
+};
+int bsk_dpair_items_round(int ni);
+bool bsk_dpair_fits(int sets, int nshell);  // registers and LDS hold a launch's shells
+int bsk_triple_dpairs_launch(const DPairArgs& a, int sets, int ni, hipStream_t s);
+size_t bsk_reduce_dpairs_bytes(int items_per_wg);
+int bsk_reduce_dpairs_launch(const double* partial, int nwg, int items_per_wg, int ntri,
+                             const int* slot, double scale, double* out, double* sums,
+                             hipStream_t s);
+// Second step of both reductions: per triangle the kRedSplit range sums of
+// its slots.
+constexpr int kRedSplit = 16;
+int bsk_reduce_tri_launch(const double* sums, int nslot, int ntri, const int* slot, double scale,
+                          double* out, hipStream_t s);
+
 // Fused z c2r + split-BF16 triple sums (zfused.hip): shell meshes with a
 // compiled kernel, at most kZMaxShells shells.
 #define BSK_ZFUSED_SIZES(X) \

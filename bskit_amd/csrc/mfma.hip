@@ -296,8 +296,6 @@ __global__ __launch_bounds__(kNT, (pair_occupancy<NI, PV, SETS, D2>())) void k_t
 // workgroups of each of kRedSplit ranges in FP64; k_reduce_tri adds, per
 // triangle, the ranges of its slots (one per launch segment of its level,
 // kPairSlots entries, -1 for none) and applies the scale and the level factor.
-constexpr int kRedSplit = 16;
-
 __global__ __launch_bounds__(256) void k_reduce_slots(const float* __restrict__ partial, int nwg,
                                                       int nslot, double* __restrict__ sums) {
   const int e = blockIdx.x * 256 + threadIdx.x, c = blockIdx.y;
@@ -461,6 +459,11 @@ int bsk_reduce_mfma_launch(const float* partial, int nwg, int items_per_wg, int 
   hipLaunchKernelGGL(k_reduce_slots, dim3((nslot + 255) / 256, kRedSplit), dim3(256), 0, s,
                      partial, nwg, nslot, sums);
   BSK_LAUNCH_CHECK();
+  return bsk_reduce_tri_launch(sums, nslot, ntri, slot, scale, out, s);
+}
+
+int bsk_reduce_tri_launch(const double* sums, int nslot, int ntri, const int* slot, double scale,
+                          double* out, hipStream_t s) {
   hipLaunchKernelGGL(k_reduce_tri, dim3((ntri + 255) / 256), dim3(256), 0, s, sums, nslot, ntri,
                      slot, scale, out);
   BSK_LAUNCH_CHECK();

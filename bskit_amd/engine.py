@@ -22,8 +22,14 @@ from . import _lib as L
 PATH_PLAIN = 'plain'      # one sweep per triangle in the shell precision
 PATH_MFMA = 'mfma'        # split-BF16 MFMA, FP32 accumulate, FP64 reduce
 PATH_BLOCKED = 'blocked'  # the plain path's FP32 sums, one sweep per block of triangles
+PATH_PAIRS64 = 'pairs64'  # FP64 MFMA, FP64 throughout
 PATH_TILED = 'tiled'      # LDS tiled VALU in the shell precision
-PATHS = (PATH_PLAIN, PATH_BLOCKED, PATH_MFMA, PATH_TILED)
+PATHS = (PATH_PLAIN, PATH_BLOCKED, PATH_MFMA, PATH_PAIRS64, PATH_TILED)
+
+# FP64 shells use the level layout from this shell mesh up: below, the one
+# launch over every cell (25 us at S = 80, 14 bins) is cheaper than up to
+# three more launches.
+F64_LEVELS_MESH = 128
 
 _MODE = {1: L.MODE_AUTO, 2: L.MODE_AAB, 3: L.MODE_ABC}
 
@@ -174,15 +180,20 @@ class PairPlan:
     """Owner of a bsk_pairs plan: the MFMA kernel's tiles for one triangle list
     (with ``levels``: the sublattice level each triangle is summed over)."""
 
-    def __init__(self, tri, nshell, mode, upload=True, levels=None):
+    def __init__(self, tri, nshell, mode, upload=True, levels=None, f64=False):
         tri = np.ascontiguousarray(np.asarray(tri, dtype=np.int32).reshape(-1, 3))
         h = ctypes.c_void_p()
         ip = ctypes.POINTER(ctypes.c_int)
-        if levels is None:
+        if levels is not None:
+            levels = np.ascontiguousarray(np.asarray(levels, dtype=np.int32).reshape(-1))
+        if f64:  # for the FP64 sums
+            L.call('bsk_pairs_create_f64', ctypes.byref(h), int(mode), int(nshell), len(tri),
+                   tri.ctypes.data_as(ip),
+                   levels.ctypes.data_as(ip) if levels is not None else None)
+        elif levels is None:
             L.call('bsk_pairs_create', ctypes.byref(h), int(mode), int(nshell), len(tri),
                    tri.ctypes.data_as(ip))
         else:
-            levels = np.ascontiguousarray(np.asarray(levels, dtype=np.int32).reshape(-1))
             L.call('bsk_pairs_create_levels', ctypes.byref(h), int(mode), int(nshell), len(tri),
                    tri.ctypes.data_as(ip), levels.ctypes.data_as(ip))
         self.handle = h
@@ -468,16 +479,17 @@ class GridEngine:
             self._tri_cache[key] = t
         return t
 
-    def pair_plan(self, tri, nshell, mode, levels=False):
+    def pair_plan(self, tri, nshell, mode, levels=False, f64=False):
         """Cached MFMA pair plan of a triangle list (host tables uploaded once);
-        levels=True sums each triangle over its sublattice level."""
+        levels=True sums each triangle over its sublattice level; f64: for the
+        FP64 sums."""
         tri = np.ascontiguousarray(np.asarray(tri, dtype=np.int32).reshape(-1, 3))
-        key = (tri.tobytes(), 'pairs', nshell, mode, bool(levels))
+        key = (tri.tobytes(), 'pairs', nshell, mode, bool(levels), bool(f64))
         r = self._tri_cache.get(key)
         if r is None:
             lv = self.triangle_levels(tri) if levels else None
             with torch.cuda.device(self.device):
-                r = PairPlan(tri, nshell, mode, levels=lv)
+                r = PairPlan(tri, nshell, mode, levels=lv, f64=f64)
             self._tri_cache[key] = r
         return r
 
@@ -504,6 +516,11 @@ class GridEngine:
     def mfma_supported(nshell, nfield, tri):
         """Whether the MFMA kernel covers this shell count / field roles."""
         return nshell <= (96 if nfield == 3 else 128)
+
+    @staticmethod
+    def pairs64_supported(nshell, nfield):
+        """Whether the FP64 pair kernel holds this many shells per field role."""
+        return nshell <= {1: 272, 2: 140, 3: 94}[nfield]
 
     def zfused_supported(self, tri):
         """Whether the fused z c2r + split-BF16 triple-sum kernel covers the
@@ -559,6 +576,13 @@ class GridEngine:
         if self.tuned_zfused_nwg:
             return self.tuned_zfused_nwg
         return int(max(1, min(512, self.S * self.S // 8)))
+
+    @staticmethod
+    def pairs64_nwg(ncell):
+        """Workgroups of the FP64 pair kernel: up to four per CU, each with at
+        least eight of its 64-cell chunks (512^3 / 32 bins: 512 workgroups 874 us,
+        768 769, 1024 744)."""
+        return int(max(8, min(1024, ncell // 512 // 8 * 8)))
 
     def plain_nchunk(self, ncell=None):
         ncell = self.ncell if ncell is None else ncell
@@ -654,6 +678,28 @@ class GridEngine:
             w = (work or self.work).get('plain', nbytes.value)
             L.call('bsk_triples_blocked', plan.handle, L.ptr(sa.data), L.ptr(sb.data),
                    L.ptr(sc.data), sa.stride, sa.sum_cells, nchunk, float(scale), L.ptr(out),
+                   L.ptr(w), s)
+            return out
+        if path == PATH_PAIRS64:
+            if any(x.fmt != L.FMT_F64 for x in sets):
+                raise ValueError('the FP64 pair path needs F64 shells')
+            lay = sa.layout
+            if any(x.layout != lay for x in sets):
+                raise ValueError('shell sets of one call need the same layout')
+            if any(x.parts is not None for x in sets):
+                raise ValueError('the FP64 pair path needs whole shells')
+            plan = self.pair_plan(tri, min(x.nb for x in sets), _MODE[nf], levels=lay is not None,
+                                  f64=True)
+            nwg = self.pairs64_nwg(sa.sum_cells) if nwg is None else int(nwg)
+            off = cells = None
+            if lay is not None:
+                off = (ctypes.c_longlong * L.LEVELS)(*lay.off)
+                cells = (ctypes.c_longlong * L.LEVELS)(*lay.ncell)
+            nbytes = L.size_out()
+            L.call('bsk_triples_mfma_workspace', plan.handle, nwg, ctypes.byref(nbytes))
+            w = (work or self.work).get('mfma', nbytes.value)
+            L.call('bsk_triples_f64', plan.handle, L.ptr(sa.data), L.ptr(sb.data), L.ptr(sc.data),
+                   sa.stride, sa.sum_cells, off, cells, None, nwg, float(scale), L.ptr(out),
                    L.ptr(w), s)
             return out
         if path == PATH_TILED:
@@ -846,6 +892,10 @@ class GridEngine:
         """Whether default shell sets of this format use the sublattice level
         layout (and MFMA sums over them the level plan)."""
         return fmt == L.FMT_BF16X2 and self.levels and self.layout is not None
+
+    def levels64(self):
+        """Whether FP64 pair sums run over the level layout of this mesh."""
+        return self.levels and self.layout is not None and self.S >= F64_LEVELS_MESH
 
     def shell_bytes(self, fmt, nb=None):
         """Device bytes of a default shell set (alloc_shells) of nb shells."""

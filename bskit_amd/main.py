@@ -301,6 +301,7 @@ class FFTBispectrum:
         key = _bins_key(kLU)
         sets = []
         meshes = self._meshes()
+        pairs64 = fmt == L.FMT_F64 and eng.pairs64_supported(eng.nb, len(self._fields))
         for fi, f in enumerate(self._fields):
             # one set of shells per field; keep the last bin set only.  Each
             # mesh is deconvolved by its own CIC window (measure_bs_fast.py
@@ -313,11 +314,13 @@ class FFTBispectrum:
                 for k in [k for k in self._shells if k[1] == fi]:
                     del self._shells[k]
                 dk = eng.forward(f, window=win)
-                s = eng.shells(dk, kind=L.KIND_DELTA, fmt=fmt,
+                out = eng.alloc_shells(fmt, eng.nb, levels=eng.levels64()) if pairs64 else None
+                s = eng.shells(dk, kind=L.KIND_DELTA, fmt=fmt, out=out,
                                dtype=torch.float32 if fmt != L.FMT_F64 else torch.float64)
                 self._shells[skey] = s
             sets.append(s)
-        path = {L.FMT_BF16X2: 'mfma', L.FMT_F32: 'blocked', L.FMT_F64: 'plain'}[fmt]
+        path = {L.FMT_BF16X2: 'mfma', L.FMT_F32: 'blocked',
+                L.FMT_F64: 'pairs64' if pairs64 else 'plain'}[fmt]
         return sets, path
 
     def _unnorm_sums(self, kLU, tri, factor):

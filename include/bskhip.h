@@ -335,6 +335,23 @@ int bsk_triples_mfma_levels_noalloc(const bsk_pairs* pairs, const uint16_t* hi_i
                                     const uint16_t* lo_k, long long shell_stride,
                                     const long long* level_off, const long long* level_ncell,
                                     int nwg, double scale, double* out_dev, void* stream);
+/* The same sums in FP64 throughout: shells of FP64 values, pair products,
+ * products with the third side and accumulation on v_mfma_f64_16x16x4.  The
+ * plan takes the lists of bsk_pairs_create (level == NULL: every triangle over
+ * the whole row, C order) or bsk_pairs_create_levels, and works with the
+ * bsk_pairs_* functions; up to 272 shells, 140 for <AAB>, 94 for <ABC>.
+ * Replaces the loop of measure_bispectrum_faster on FP64 grids
+ * (bskit/main.py:1871-1882) and the sums of measure_gridinfo_faster
+ * (:2024-2064).  weight: optional FP64 weight per cell (auto spectra), each
+ * product multiplied by it.  level_off / level_ncell NULL: ncell cells in C
+ * order, a multiple of 64.  work: bsk_triples_mfma_workspace(pairs, nwg). */
+int bsk_pairs_create_f64(bsk_pairs** pairs, int mode, int nshell, int ntri, const int* tri_host,
+                         const int* level);
+int bsk_triples_f64(const bsk_pairs* pairs, const double* f_i, const double* f_j,
+                    const double* f_k, long long shell_stride, long long ncell,
+                    const long long* level_off, const long long* level_ncell,
+                    const double* weight, int nwg, double scale, double* out_dev, void* work,
+                    void* stream);
 /* out_dev == NULL in bsk_triples_mfma leaves the per-workgroup partials in
  * work; bsk_triples_mfma_reduce then sums them in FP64 into out_dev (the
  * same result as one call with out_dev; it uses the tail of work, after the
