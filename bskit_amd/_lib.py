@@ -58,6 +58,9 @@ _SIGS = {
     'bsk_pairs_create_f64': [ctypes.POINTER(_vp), _c_int, _c_int, _c_int, _int_p, _int_p],
     'bsk_triples_f64': [_vp, _vp, _vp, _vp, _c_ll, _c_ll, ctypes.POINTER(_c_ll),
                         ctypes.POINTER(_c_ll), _vp, _c_int, _c_double, _vp, _vp, _vp],
+    'bsk_gridinfo_pairs': [ctypes.POINTER(_vp), _c_int, _c_int, _int_p],
+    'bsk_gridinfo_layout': [_vp, _c_int, _c_int, ctypes.POINTER(_c_ll), _c_size_p],
+    'bsk_gridinfo_shells': [_vp, _c_int, _c_int, _vp, _c_ll, _vp, _vp, _vp],
     'bsk_blocked_create': [ctypes.POINTER(_vp), _c_int, _c_int, _c_int, _int_p],
     'bsk_blocked_upload': [_vp],
     'bsk_blocked_destroy': [_vp],

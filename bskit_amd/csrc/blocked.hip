@@ -320,7 +320,7 @@ struct Tri {
 struct bsk_blocked {
   int ntri = 0, nrow = 0;
   std::vector<int> tri;  // the list as given, for k_triple_plain
-  int* d_tri = nullptr;
+  int* d_tri = nullptr;  // owns the block of all device tables
   BlockTables t4, t2;  // blocks of 4 and of 2 shells
 };
 
@@ -454,31 +454,6 @@ void make_tables(BlockTables& t, const int set[3], const std::vector<Tri>& tri) 
   }
 }
 
-int upload_ints(int** dst, const std::vector<int>& v) {
-  BSK_HIP_CHECK(hipMalloc(dst, sizeof(int) * std::max<size_t>(v.size(), 1)));
-  if (!v.empty())
-    BSK_HIP_CHECK(hipMemcpy(*dst, v.data(), sizeof(int) * v.size(), hipMemcpyHostToDevice));
-  return BSK_OK;
-}
-
-int upload_tables(BlockTables& t) {
-  int rc = upload_ints(&t.d_tabs, t.tabs);
-  if (!rc) rc = upload_ints(&t.d_rows, t.rows);
-  if (!rc) rc = upload_ints(&t.d_entry, t.entry);
-  return rc;
-}
-
-void free_device(bsk_blocked* q) {
-  for (BlockTables* t : {&q->t4, &q->t2}) {
-    (void)hipFree(t->d_tabs);
-    (void)hipFree(t->d_rows);
-    (void)hipFree(t->d_entry);
-    t->d_tabs = t->d_rows = t->d_entry = nullptr;
-  }
-  (void)hipFree(q->d_tri);
-  q->d_tri = nullptr;
-}
-
 // Rows of partial sums held at a time: longer lists run in several launches.
 constexpr int kRowBatch = 16384;
 
@@ -589,16 +564,15 @@ int bsk_blocked_upload(bsk_blocked* q) {
     return BSK_EINVAL;
   }
   if (q->d_tri) return BSK_OK;
-  int rc = upload_tables(q->t4);
-  if (!rc) rc = upload_tables(q->t2);
-  if (!rc) rc = upload_ints(&q->d_tri, q->tri);
-  if (rc) free_device(q);
-  return rc;
+  return bsk_upload_tables({&q->tri, &q->t4.tabs, &q->t4.rows, &q->t4.entry, &q->t2.tabs,
+                            &q->t2.rows, &q->t2.entry},
+                           {&q->d_tri, &q->t4.d_tabs, &q->t4.d_rows, &q->t4.d_entry, &q->t2.d_tabs,
+                            &q->t2.d_rows, &q->t2.d_entry});
 }
 
 int bsk_blocked_destroy(bsk_blocked* q) {
   if (!q) return BSK_OK;
-  free_device(q);
+  (void)hipFree(q->d_tri);
   delete q;
   return BSK_OK;
 }

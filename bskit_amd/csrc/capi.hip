@@ -273,6 +273,28 @@ int check_plan(const bsk_plan* p) {
 
 }  // namespace
 
+int bsk_upload_tables(const std::vector<const std::vector<int>*>& tables,
+                      const std::vector<int**>& where) {
+  std::vector<size_t> at;
+  size_t n = 0;
+  for (const auto* t : tables) {
+    at.push_back(n);
+    n += (t->size() + 3) & ~(size_t)3;
+  }
+  std::vector<int> all(std::max<size_t>(n, 4), 0);
+  for (size_t k = 0; k < tables.size(); ++k)
+    std::copy(tables[k]->begin(), tables[k]->end(), all.begin() + at[k]);
+  int* d = nullptr;
+  BSK_HIP_CHECK(hipMalloc(&d, sizeof(int) * all.size()));
+  const hipError_t e = hipMemcpy(d, all.data(), sizeof(int) * all.size(), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    (void)hipFree(d);
+    BSK_HIP_CHECK(e);
+  }
+  for (size_t k = 0; k < tables.size(); ++k) *where[k] = d + at[k];
+  return BSK_OK;
+}
+
 bool bsk_fft_size_supported(int N) {
   switch (N) {
 #define X(n) case n:
@@ -797,7 +819,7 @@ struct bsk_pairs {
   int item_total = 0;  // distinct items: partial positions per workgroup
   std::vector<int> slot;  // [ntri][kParts]: each triangle's slot per segment, -1 for none
   std::vector<int> h_items, h_outpos, h_pairs;
-  int* d_items = nullptr;   // per launch [waves * ni of its segment]
+  int* d_items = nullptr;   // per launch [waves * ni of its segment]; owns the tables' block
   int* d_outpos = nullptr;  // the same shape
   int* d_pairs = nullptr;   // [ntile + 1][16]
   int* d_slot = nullptr;    // [ntri][kParts]
@@ -951,13 +973,6 @@ std::vector<Role> assign_roles_cover(int ntri, const int* tri) {
   return r;
 }
 
-int upload(int** dst, const std::vector<int>& v) {
-  BSK_HIP_CHECK(hipMalloc(dst, sizeof(int) * std::max<size_t>(v.size(), 1)));
-  if (!v.empty())
-    BSK_HIP_CHECK(hipMemcpy(*dst, v.data(), sizeof(int) * v.size(), hipMemcpyHostToDevice));
-  return BSK_OK;
-}
-
 // One level's share of a pair plan: role choice, tiles and units (a tile
 // with at most `cap` of its kb blocks; each unit forms the tile's pair
 // products once), in absolute shell indices.
@@ -970,8 +985,9 @@ struct LevelPlan {
   int lo = 0, hi = 0;  // shells used: [lo, hi)
 };
 
+// given: the roles of every triangle of tri, or null to choose them.
 LevelPlan plan_level(int mode, int nkb, int cap, const std::vector<int>& idx, const int* tri,
-                     bool f64) {
+                     bool f64, const std::vector<Role>* given = nullptr) {
   LevelPlan lp;
   lp.tri = idx;
   std::vector<int> sub((size_t)3 * idx.size());
@@ -986,8 +1002,13 @@ LevelPlan plan_level(int mode, int nkb, int cap, const std::vector<int>& idx, co
   const int ntri = (int)idx.size();
   // role assignment: the fixed roles of <AAB>/<ABC>; for auto spectra the
   // choice of the pair sides that needs the fewest items
-  const int nopt = mode == BSK_MODE_AUTO ? 4 : 1;
+  // (FP64: the two largest, whatever the list)
+  const int nopt = given ? 0 : (mode == BSK_MODE_AUTO && !f64 ? 4 : 1);
   bool first = true;
+  if (given) {
+    for (int t : idx) lp.roles.push_back((*given)[t]);
+    lp.tiles = build_tiles(lp.roles, false);
+  }
   for (int o = 0; o < nopt; ++o) {
     std::vector<Role> r =
         o == 3 ? assign_roles_cover(ntri, sub.data()) : assign_roles(mode, o, ntri, sub.data());
@@ -1067,7 +1088,8 @@ std::vector<std::vector<int>> bin_units(const std::vector<unsigned>& mask, int c
 }
 
 int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri,
-                 const int* level, const char* fn, bool f64 = false) {
+                 const int* level, const char* fn, bool f64 = false,
+                 const std::vector<Role>* roles = nullptr) {
   if (!out || nshell < 1 || mode < 0 || mode > 2 || ntri < 0 || (ntri && !tri)) {
     bsk_set_error("%s: invalid argument", fn);
     return BSK_EINVAL;
@@ -1118,7 +1140,9 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
   for (int p = 0; p < kParts; ++p) {
     const unsigned lv = kPartLevels[p] & present;
     if (!lv) continue;
-    if (!segs.empty() && segs.back().lv == lv && (segs.back().parts >> (p - 1) & 1))
+    // (FP64 sums keep every part a segment, so that the order in which a
+    // triangle's cells are added does not depend on the rest of the list)
+    if (!segs.empty() && segs.back().lv == lv && (segs.back().parts >> (p - 1) & 1) && !(f64 && level))
       segs.back().parts |= 1 << p;
     else
       segs.push_back({1 << p, lv});
@@ -1137,7 +1161,7 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
     for (int L = 0; L < BSK_LEVELS; ++L)
       if (segs[g].lv >> L & 1) sel.insert(sel.end(), idx[L].begin(), idx[L].end());
     std::sort(sel.begin(), sel.end());
-    lp[g] = plan_level(mode, nkb, cap, sel, tri, f64);
+    lp[g] = plan_level(mode, nkb, cap, sel, tri, f64, roles);
     tile0[g + 1] = tile0[g] + (int)lp[g].tiles.tile_mask.size();
   }
   const int ntile = tile0[nseg];
@@ -1180,21 +1204,7 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
       sp[g].npass = 1;
       sp[g].bins.assign(W, {});
     } else if (f64) {
-      // lists on W / rep waves, replicated rep times, each replica running
-      // every rep-th K step: the count that leaves the fullest wave the least
-      double best = 0.0;
-      for (int rep : {1, 2, 4, 8}) {
-        int np = 0, m2 = 1;
-        auto b2 = bin_units(sp[g].unit_mask, cap, W / rep, &np, &m2, 0);
-        const double t = (double)np * bsk_dpair_items_round(m2) / rep;
-        if (rep > 1 && (np > 1 || t >= best)) continue;
-        best = t;
-        ml = m2;
-        sp[g].npass = np;
-        sp[g].rep = rep;
-        sp[g].bins.clear();
-        for (int r = 0; r < rep; ++r) sp[g].bins.insert(sp[g].bins.end(), b2.begin(), b2.end());
-      }
+      sp[g].bins = bin_units(sp[g].unit_mask, cap, W, &sp[g].npass, &ml, 0);
     } else {
       sp[g].bins = bin_units(sp[g].unit_mask, cap, W, &sp[g].npass, &ml);
       // few items (a plan over levels): lists on W / rep waves, replicated
@@ -1383,26 +1393,13 @@ int bsk_pairs_upload(bsk_pairs* q) {
     return BSK_EINVAL;
   }
   if (q->d_items) return BSK_OK;
-  int rc = upload(&q->d_items, q->h_items);
-  if (!rc) rc = upload(&q->d_outpos, q->h_outpos);
-  if (!rc) rc = upload(&q->d_pairs, q->h_pairs);
-  if (!rc) rc = upload(&q->d_slot, q->slot);
-  if (rc) {
-    (void)hipFree(q->d_items);
-    (void)hipFree(q->d_outpos);
-    (void)hipFree(q->d_pairs);
-    (void)hipFree(q->d_slot);
-    q->d_items = q->d_outpos = q->d_pairs = q->d_slot = nullptr;
-  }
-  return rc;
+  return bsk_upload_tables({&q->h_items, &q->h_outpos, &q->h_pairs, &q->slot},
+                           {&q->d_items, &q->d_outpos, &q->d_pairs, &q->d_slot});
 }
 
 int bsk_pairs_destroy(bsk_pairs* q) {
   if (!q) return BSK_OK;
-  (void)hipFree(q->d_items);
-  (void)hipFree(q->d_outpos);
-  (void)hipFree(q->d_pairs);
-  (void)hipFree(q->d_slot);
+  (void)hipFree(q->d_items);  // the block of all tables
   delete q;
   return BSK_OK;
 }
@@ -1745,6 +1742,102 @@ int bsk_triples_mfma_reduce(const bsk_pairs* q, int nwg, double scale, double* o
                                 as_stream(stream));
 }
 
+// --------------------------------------------------------------- grid info
+int bsk_gridinfo_pairs(bsk_pairs** out, int nb, int ntri, const int* tri) {
+  const char* fn = "bsk_gridinfo_pairs";
+  if (!out || nb < 1 || ntri < 0 || ntri > INT_MAX / 12 || (ntri && !tri)) {
+    bsk_set_error("%s: invalid argument", fn);
+    return BSK_EINVAL;
+  }
+  for (int t = 0; t < 3 * ntri; ++t)
+    if (tri[t] < 0 || tri[t] >= nb) {
+      bsk_set_error("%s: triangle %d has a shell index out of range", fn, t / 3);
+      return BSK_EINVAL;
+    }
+  // pairs for the unit-shell sums, then per triangle each side's |k| shell in
+  // the place of its unit shell: on the third side where it may (the pair
+  // products are shared), else on the pair side
+  const std::vector<Role> base = assign_roles_cover(ntri, tri);
+  std::vector<Role> roles((size_t)4 * ntri);
+  std::vector<int> list((size_t)12 * ntri);
+  for (int t = 0; t < ntri; ++t) {
+    const Role r = base[t];
+    roles[4 * (size_t)t] = r;
+    for (int e = 0; e < 3; ++e) {
+      Role& q = roles[4 * (size_t)t + 1 + e] = r;
+      const int v = tri[3 * t + e];
+      if (r.c == v) q.c += nb;
+      else if (r.a == v) q.a += nb;
+      else q.b += nb;
+    }
+    for (int s = 0; s < 4; ++s) {
+      const Role& q = roles[4 * (size_t)t + s];
+      int* l = &list[12 * (size_t)t + 3 * s];
+      l[0] = q.a, l[1] = q.b, l[2] = q.c;
+    }
+  }
+  return pairs_create(out, BSK_MODE_AUTO, 2 * nb, 4 * ntri, list.data(), nullptr, fn, true, &roles);
+}
+
+static int gridinfo_args(const bsk_plan* p, int x0, int x1, GridInfoArgs& a, size_t* bytes) {
+  if (x0 < 0 || x1 <= x0 || x1 > p->S / 2 + 1 || p->S % 2) {
+    bsk_set_error("bsk_gridinfo: planes [%d, %d) of 0..%d, even shell mesh", x0, x1, p->S / 2);
+    return BSK_EINVAL;
+  }
+  a = {};
+  a.S = p->S;
+  a.mm = std::min(p->m, p->S / 2);
+  a.nb = p->nbin;
+  a.x0 = x0;
+  a.x1 = x1;
+  a.NP = (a.mm + 8) & ~7;
+  a.P = (a.mm + 1) * a.NP;
+  a.XP = (p->S / 2 + 8) & ~7;
+  a.n2lo = p->d_lo;
+  a.n2hi = p->d_hi;
+  a.kf = 2.0 * M_PI / p->box;
+  auto tri2 = [](long long v) { return v * (v + 1) / 2; };
+  auto tri3 = [](long long v) { return v * (v + 1) * (v + 2) / 6; };
+  a.cells = tri3(x1) - tri3(x0);
+  a.padded = (a.cells + kDPairChunk - 1) / kDPairChunk * kDPairChunk;
+  const size_t tab = (size_t)a.NP * a.XP;
+  const size_t g = (size_t)2 * a.nb * (x1 - x0) * a.P;
+  const size_t h = (size_t)2 * a.nb * (size_t)(tri2(x1) - tri2(x0)) * a.NP;
+  if (bytes) *bytes = sizeof(double) * (2 * tab + g + h);
+  return BSK_OK;
+}
+
+int bsk_gridinfo_layout(const bsk_plan* p, int x0, int x1, long long* ncell, size_t* work_bytes) {
+  if (int rc = check_plan(p)) return rc;
+  if (!ncell || !work_bytes) {
+    bsk_set_error("bsk_gridinfo_layout: null output");
+    return BSK_EINVAL;
+  }
+  GridInfoArgs a;
+  if (int rc = gridinfo_args(p, x0, x1, a, work_bytes)) return rc;
+  *ncell = a.padded;
+  return BSK_OK;
+}
+
+int bsk_gridinfo_shells(bsk_plan* p, int x0, int x1, double* shells, long long shell_stride,
+                        double* weight, void* work, void* stream) {
+  if (int rc = check_plan(p)) return rc;
+  GridInfoArgs a;
+  if (int rc = gridinfo_args(p, x0, x1, a, nullptr)) return rc;
+  if (!shells || !weight || !work || shell_stride < a.padded || p->nbin > 65535) {
+    bsk_set_error("bsk_gridinfo_shells: invalid argument");
+    return BSK_EINVAL;
+  }
+  a.stride = shell_stride;
+  a.f = shells;
+  a.weight = weight;
+  a.cn = reinterpret_cast<double*>(work);
+  a.cx = a.cn + (size_t)a.NP * a.XP;
+  a.g = a.cx + (size_t)a.NP * a.XP;
+  a.h = a.g + (size_t)2 * a.nb * (x1 - x0) * a.P;
+  return bsk_gridinfo_launch(shell_tw(p, 0.0), a, as_stream(stream));
+}
+
 // ------------------------------------------------------------------ FP64
 int bsk_pairs_create_f64(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri,
                          const int* level) {
@@ -1794,7 +1887,6 @@ int bsk_triples_f64(const bsk_pairs* q, const double* f_i, const double* f_j, co
     a.koff = w0 % 16;
     a.nkb = (a.koff + wn + 15) / 16;
     a.ncell = pend[lp] - pbeg[fp];
-    a.rep = q->seg_rep[g];
     const int ni = q->seg_ni[g], np = q->seg_pass[g];
     const bool fold = np > 1 && nwg % 8 == 0;
     a.npass = fold ? np : 1;

@@ -10,11 +10,12 @@
 // a segment and the shells are read once; a register-blocked sum of single
 // triangles (blocked.hip's scheme in FP64) holds 64 triangles a wave and read
 // the shells 13 times: 5.0 ms at 512^3 / 32 bins, one sweep per triangle 84 ms,
-// this 0.74 ms over the levels (2.1 without them).  FP64 MFMA and FP64 VALU
+// this 0.90 ms over the levels (1.95 without them).  FP64 MFMA and FP64 VALU
 // have the same peak on gfx950 (72 TFLOP/s measured with a large matrix
-// product) and share issue time, so what bounds it is the MFMAs (0.52 ms of
-// the 0.74 at 2.17 GHz) plus every VALU instruction between them: the K loop
-// is rolled with one address add per LDS read.
+// product) and share issue time, so what bounds it is the MFMAs (0.55 ms of
+// the 0.90 at 2.17 GHz), every VALU instruction between them (the K loop is
+// rolled with one address add per LDS read) and, in the thin segments, the
+// latency of one wave's K steps.
 //
 // Workgroup: eight waves over a contiguous range of 64-cell chunks; per chunk
 // the staged shells' rows go from HBM through registers (loaded one chunk
@@ -22,8 +23,16 @@
 // reads of 16 arbitrary rows best).  Lane (col, grp) of a wave reads cells 2
 // grp and 2 grp + 1 of an eight-cell K step, of its pair's two rows and of its
 // third-side row; the first MFMA takes the even cells, the second the odd
-// ones.  A segment with few items replicates its wave lists over 2, 4 or 8
-// wave groups that take alternate K steps.
+// ones.  Workgroups of a CU turn the lists by one wave each, so that the items
+// of a thin segment (or the ninth of nine) are on different SIMDs.
+//
+// A triangle's sum does not depend on the list it is summed with: its pair is
+// its two largest shells (28 items at 512^3 / 32 bins; the greedy cover of the
+// split-BF16 plans needs 26), every part of the level layout is a segment of
+// its own, the workgroups' cell ranges follow from the mesh, and one wave adds
+// all K steps of an item in order (lists that share an item's K steps between
+// waves are faster where few items meet many cells, 0.74 ms for the list above,
+// but how many share them follows from the list).
 #include <algorithm>
 
 #include "launch.h"
@@ -53,29 +62,25 @@ __host__ __device__ inline Rows lds_rows(int sets, int n0, int n1, int nkb) {
   return r;
 }
 
-template <int NI, int PV, int SETS, bool WT>
-__global__ __launch_bounds__(kNT, 2) void k_triple_dpairs(DPairArgs a) {
-  extern __shared__ __attribute__((aligned(16))) double smem[];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int rep = a.rep, rgrp = wave / (kW / rep);
+// The chunks of one workgroup for a wave with CNT items (the other waves of
+// the workgroup may run another count: all run the same barriers).  Straight
+// code for CNT items: with a branch around an item's MFMAs the compiler copies
+// the accumulators at every join.
+template <int CNT, int PV, int SETS, bool WT>
+BSK_DEV void run_items(const DPairArgs& a, double* smem, const int* items, const int* outpos,
+                       int lw) {
   const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
   const Rows R = lds_rows(SETS, a.nsh, a.nsh, a.nkb);
   // LDS row of staged shell 0 of each set: the third side's blocks are
   // 16-aligned, so it starts at koff
   const int s0 = SETS == 1 ? a.koff : 0, s1 = R.r1, s2 = R.r2 + a.koff;
-
-  int lw = blockIdx.x, pass = 0;  // cell range and item-list pass (see PairArgs)
-  if (a.npass > 1) {
-    pass = (blockIdx.x >> 3) % a.npass;
-    lw = (blockIdx.x / (8 * a.npass)) * 8 + (blockIdx.x & 7);
-  }
-  const int* items = a.items + pass * a.pass_stride + wave * NI;
-  const int* outpos = a.outpos + pass * a.pass_stride + wave * NI;
   // per item: descriptor, this lane's offsets of its pair rows (padding rows
   // read row 0: their sums are never read) and of its third-side row
-  int desc[NI], oi[NI], oj[NI], ok[NI];
+  constexpr int NC = CNT ? CNT : 1;
+  int desc[NC], oi[NC], oj[NC], ok[NC];
+  d4 acc[NC];
 #pragma unroll
-  for (int s = 0; s < NI; ++s) {
+  for (int s = 0; s < CNT; ++s) {
     desc[s] = __builtin_amdgcn_readfirstlane(items[s]);
     const int pr = a.pairs[(desc[s] & 0xffff) * 16 + col];
     const int ra = pr & 0xffff, rb = (pr >> 16) & 0xffff;
@@ -83,16 +88,14 @@ __global__ __launch_bounds__(kNT, 2) void k_triple_dpairs(DPairArgs a) {
     oi[s] = (s0 + ia) * kLD + 2 * grp;
     oj[s] = ((SETS == 3 ? s1 : s0) + ib) * kLD + 2 * grp;
     ok[s] = (R.r2 + 16 * ((desc[s] >> 16) & 0xff) + col) * kLD + 2 * grp;
+    acc[s] = d4{0.0, 0.0, 0.0, 0.0};
   }
-  d4 acc[NI];
-#pragma unroll
-  for (int s = 0; s < NI; ++s) acc[s] = d4{0.0, 0.0, 0.0, 0.0};
 
   // staging: segment v = thread + k kNT is 16 bytes of staged row v / kSEG:
   // the shells of set 0, then 1, then 2, then the weights
   const int n = a.nsh, nrow = SETS * n + (WT ? 1 : 0);
-  const long long nch = a.ncell / kCK;
-  const long long ch0 = nch * lw / a.nwg, ch1 = nch * (lw + 1) / a.nwg;
+  const int nch = (int)(a.ncell / kCK);
+  const int ch0 = (int)((long long)nch * lw / a.nwg), ch1 = (int)((long long)nch * (lw + 1) / a.nwg);
   const double* src[PV];
   int dst[PV];
 #pragma unroll
@@ -103,7 +106,7 @@ __global__ __launch_bounds__(kNT, 2) void k_triple_dpairs(DPairArgs a) {
     const bool wt = WT && row == nrow - 1;
     const double* base = set == 0 ? a.f[0] : (SETS == 3 && set == 1 ? a.f[1] : a.f[2]);
     const int lrow = set == 0 ? s0 : (SETS == 3 && set == 1 ? s1 : s2);
-    src[k] = wt ? a.weight + 2 * sg + ch0 * kCK : base + sh * a.stride + 2 * sg + ch0 * kCK;
+    src[k] = (wt ? a.weight : base + sh * a.stride) + 2 * sg + (long long)ch0 * kCK;
     dst[k] = row < nrow ? (wt ? R.rw : lrow + sh) * kLD + 2 * sg : -1;
   }
   d2 pre[PV];
@@ -115,65 +118,69 @@ __global__ __launch_bounds__(kNT, 2) void k_triple_dpairs(DPairArgs a) {
     }
   };
   if (ch0 < ch1) fetch();
-  for (long long ch = ch0; ch < ch1; ++ch) {
+  for (int ch = ch0; ch < ch1; ++ch) {
     __syncthreads();  // every wave is done with the previous chunk
 #pragma unroll
     for (int k = 0; k < PV; ++k)
       if (dst[k] >= 0) *reinterpret_cast<d2*>(smem + dst[k]) = pre[k];
     __syncthreads();
     if (ch + 1 < ch1) fetch();  // the next chunk's loads overlap this one's math
-    for (int ks = rgrp; ks < kSteps; ks += rep) {
+    if (CNT == 0) continue;
+#pragma unroll 1
+    for (int ks = 0; ks < kSteps; ++ks) {
       int o = 8 * ks;
       asm("" : "+s"(o));  // keeps one add per read, not an induction variable per row
       const double* f = smem + o;
       d2 p = {0.0, 0.0};
 #pragma unroll
-      for (int s = 0; s < NI; ++s) {
-        if (desc[s] & (1 << 29)) continue;  // uniform: padding item
+      for (int s = 0; s < CNT; ++s) {
         const d2 z = *reinterpret_cast<const d2*>(f + ok[s]);
-        if (s == 0 || desc[s] < 0) {        // uniform: new tile, new pair products
+        if (s == 0 || desc[s] < 0) {  // uniform: new tile, new pair products
           const d2 x = *reinterpret_cast<const d2*>(f + oi[s]);
           const d2 y = *reinterpret_cast<const d2*>(f + oj[s]);
-          p = {x.x * y.x, x.y * y.y};
-          if (WT) {
-            const d2 w = *reinterpret_cast<const d2*>(f + R.rw * kLD + 2 * grp);
-            p = {p.x * w.x, p.y * w.y};
-          }
+          p = x * y;
+          if (WT) p *= *reinterpret_cast<const d2*>(f + R.rw * kLD + 2 * grp);
         }
         acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(p.x, z.x, acc[s], 0, 0, 0);
         acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(p.y, z.y, acc[s], 0, 0, 0);
       }
     }
   }
-  // replicas of a wave's list ran other K steps: the first adds theirs
-  // through LDS and stores
-  if (rep > 1) {
-    const int wpr = kW / rep, wl = wave % wpr;
-    for (int g = 1; g < rep; ++g) {
-      __syncthreads();
-      if (rgrp == g)
-#pragma unroll
-        for (int s = 0; s < NI; ++s)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) smem[((wl * NI + s) * 4 + r) * 64 + lane] = acc[s][r];
-      __syncthreads();
-      if (rgrp == 0)
-#pragma unroll
-        for (int s = 0; s < NI; ++s)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[s][r] += smem[((wl * NI + s) * 4 + r) * 64 + lane];
-    }
-    if (rgrp) return;
-  }
   // C[row][col]: register r of lane group grp is row 4 r + grp
   double* const out = a.partial + (long long)lw * a.item_total * 256;
 #pragma unroll
-  for (int s = 0; s < NI; ++s) {
+  for (int s = 0; s < CNT; ++s) {
     const int pos = __builtin_amdgcn_readfirstlane(outpos[s]);
-    if (pos < 0) continue;  // uniform
 #pragma unroll
     for (int r = 0; r < 4; ++r) out[(long long)pos * 256 + (4 * r + grp) * 16 + col] = acc[s][r];
   }
+}
+
+template <int CNT, int PV, int SETS, bool WT>
+BSK_DEV void run_count(int cnt, const DPairArgs& a, double* smem, const int* items,
+                       const int* outpos, int lw) {
+  if (cnt >= CNT)  // uniform per wave
+    run_items<CNT, PV, SETS, WT>(a, smem, items, outpos, lw);
+  else if constexpr (CNT > 0)
+    run_count<CNT - 1, PV, SETS, WT>(cnt, a, smem, items, outpos, lw);
+}
+
+template <int NI, int PV, int SETS, bool WT>
+__global__ __launch_bounds__(kNT, NI <= 4 && PV <= 10 ? 4 : 2) void k_triple_dpairs(DPairArgs a) {
+  extern __shared__ __attribute__((aligned(16))) double smem[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int lw = blockIdx.x, pass = 0;  // cell range and item-list pass (see PairArgs)
+  if (a.npass > 1) {
+    pass = (blockIdx.x >> 3) % a.npass;
+    lw = (blockIdx.x / (8 * a.npass)) * 8 + (blockIdx.x & 7);
+  }
+  const int list = (wave + (lw >> 8)) & (kW - 1);
+  const int* items = a.items + pass * a.pass_stride + list * NI;
+  int cnt = 0;  // the list's items (padding follows them)
+#pragma unroll
+  for (int s = 0; s < NI; ++s)
+    cnt += __builtin_amdgcn_readfirstlane(items[s]) & (1 << 29) ? 0 : 1;
+  run_count<NI, PV, SETS, WT>(cnt, a, smem, items, a.outpos + pass * a.pass_stride + list * NI, lw);
 }
 
 template <int NI, int PV, int SETS>
@@ -202,11 +209,8 @@ int launch(const DPairArgs& a, size_t lds, hipStream_t s) {
 template <int PV, int SETS>
 int launch_ni(const DPairArgs& a, int ni, size_t lds, hipStream_t s) {
   switch (ni) {
-    case 1: return launch<1, PV, SETS>(a, lds, s);
     case 2: return launch<2, PV, SETS>(a, lds, s);
-    case 3: return launch<3, PV, SETS>(a, lds, s);
     case 4: return launch<4, PV, SETS>(a, lds, s);
-    case 6: return launch<6, PV, SETS>(a, lds, s);
     case 8: return launch<8, PV, SETS>(a, lds, s);
   }
   bsk_set_error("FP64 pair sums: %d items per wave not compiled", ni);
@@ -240,7 +244,7 @@ __global__ __launch_bounds__(256) void k_reduce_dslots(const double* __restrict_
 
 }  // namespace
 
-int bsk_dpair_items_round(int ni) { return ni <= 4 ? std::max(ni, 1) : (ni <= 6 ? 6 : (ni <= 8 ? 8 : 0)); }
+int bsk_dpair_items_round(int ni) { return ni <= 2 ? 2 : (ni <= 4 ? 4 : (ni <= 8 ? 8 : 0)); }
 
 bool bsk_dpair_fits(int sets, int nshell) {
   const int nkb = (nshell + 15) / 16 + 1;  // a window may start inside a block
@@ -253,16 +257,12 @@ int bsk_triple_dpairs_launch(const DPairArgs& a, int sets, int ni, hipStream_t s
     bsk_set_error("FP64 pair sums: cells in multiples of %d, even stride, nwg > 0", kCK);
     return BSK_EINVAL;
   }
-  if (a.npass < 1 || (a.npass > 1 && (a.nwg % 8 || a.rep != 1))) {
-    bsk_set_error("FP64 pair sums: folded passes need nwg a multiple of 8 and no replicas");
-    return BSK_EINVAL;
-  }
-  if (a.rep != 1 && a.rep != 2 && a.rep != 4 && a.rep != 8) {
-    bsk_set_error("FP64 pair sums: %d replicas (1, 2, 4 or 8)", a.rep);
+  if (a.npass < 1 || (a.npass > 1 && a.nwg % 8)) {
+    bsk_set_error("FP64 pair sums: folded passes need nwg a multiple of 8");
     return BSK_EINVAL;
   }
   const size_t rows = (size_t)lds_rows(sets, a.nsh, a.nsh, a.nkb).rw + (a.weight ? 1 : 0);
-  const size_t lds = std::max(rows * kLD * 8, a.rep > 1 ? (size_t)(kW / a.rep) * ni * 256 * 8 : 0);
+  const size_t lds = rows * kLD * 8;
   const int pv = ((sets * a.nsh + (a.weight ? 1 : 0)) * kSEG + kNT - 1) / kNT;
   if (lds > 160 * 1024) {
     bsk_set_error("FP64 pair sums: %d shells exceed the kernel's staging", a.nsh);

@@ -1,5 +1,7 @@
 // Internal host-side launch API shared by the translation units.
 #pragma once
+#include <vector>
+
 #include "common.h"
 #include "fft_passes.h"
 
@@ -9,6 +11,12 @@
   X(16) X(24) X(32) X(40) X(48) X(64) X(72) X(80) X(96) X(120) X(128) X(144) X(160)       \
   X(192) X(200) X(216) X(240) X(256) X(288) X(320) X(384) X(400) X(432) X(480) X(512)    \
   X(576) X(640) X(768) X(1024)
+
+// Host integer tables in one device block (one allocation and one copy per
+// plan): the tables' device addresses go to where[k], each 16-byte aligned;
+// where[0] owns the block (hipFree).
+int bsk_upload_tables(const std::vector<const std::vector<int>*>& tables,
+                      const std::vector<int**>& where);
 
 bool bsk_fft_size_supported(int N);
 // Smallest supported mesh size strictly greater than n (0 if none).
@@ -117,7 +125,6 @@ struct DPairArgs {
   int nwg;
   const int* items;
   const int* outpos;
-  int rep;                // replicas of the wave lists (1, 2, 4, 8)
   const int* pairs;
   double* partial;        // [nwg][item_total][256]
   int item_total;
@@ -162,6 +169,24 @@ struct ZArgs {
 size_t bsk_zrows_lds_bytes(int S, int nsh, int nkb);
 int bsk_triple_zrows_launch_v0(const ZArgs& a, int S, int ni, hipStream_t s);
 int bsk_triple_zrows_launch_v1(const ZArgs& a, int S, int ni, hipStream_t s);
+
+// Unit and |k| shells on the symmetry wedge (gridinfo.hip), planes [x0, x1).
+struct GridInfoArgs {
+  int S, mm, nb;        // shell mesh, largest component of a mode, shells
+  int x0, x1;
+  int P, NP, XP;        // entries of an (ny, nz) plane; row lengths over n and over x
+  const int* n2lo;
+  const int* n2hi;
+  double kf;
+  long long cells, padded, stride;  // wedge cells of the slab
+  double* cn;           // [NP][XP]
+  double* cx;           // [XP][NP]
+  double* g;            // [2][nb][x1 - x0][P]
+  double* h;            // [2][nb][rows][NP]
+  double* f;            // [2 nb][stride]
+  double* weight;       // [padded]
+};
+int bsk_gridinfo_launch(const cplx<double>* tw, const GridInfoArgs& a, hipStream_t s);
 
 // Power spectrum sums (spectrum.hip).
 int bsk_spectrum_launch(int dtype, const void* dk, Geom g, int N, const int* n2lo,

@@ -27,9 +27,10 @@ PATH_TILED = 'tiled'      # LDS tiled VALU in the shell precision
 PATHS = (PATH_PLAIN, PATH_BLOCKED, PATH_MFMA, PATH_PAIRS64, PATH_TILED)
 
 # FP64 shells use the level layout from this shell mesh up: below, the one
-# launch over every cell (25 us at S = 80, 14 bins) is cheaper than up to
-# three more launches.
-F64_LEVELS_MESH = 128
+# launch over every cell is cheaper than up to three more launches (shells and
+# sums, levels against C order: S = 64 / 8 bins 61 / 52 us, 96 / 14 bins <AAB>
+# 186 / 220, 160 / 16 bins 462 / 619).
+F64_LEVELS_MESH = 96
 
 _MODE = {1: L.MODE_AUTO, 2: L.MODE_AAB, 3: L.MODE_ABC}
 
@@ -180,13 +181,16 @@ class PairPlan:
     """Owner of a bsk_pairs plan: the MFMA kernel's tiles for one triangle list
     (with ``levels``: the sublattice level each triangle is summed over)."""
 
-    def __init__(self, tri, nshell, mode, upload=True, levels=None, f64=False):
+    def __init__(self, tri, nshell, mode, upload=True, levels=None, f64=False, gridinfo=False):
         tri = np.ascontiguousarray(np.asarray(tri, dtype=np.int32).reshape(-1, 3))
         h = ctypes.c_void_p()
         ip = ctypes.POINTER(ctypes.c_int)
         if levels is not None:
             levels = np.ascontiguousarray(np.asarray(levels, dtype=np.int32).reshape(-1))
-        if f64:  # for the FP64 sums
+        if gridinfo:  # four FP64 sums per triangle over unit and |k| shells
+            L.call('bsk_gridinfo_pairs', ctypes.byref(h), int(nshell), len(tri),
+                   tri.ctypes.data_as(ip))
+        elif f64:  # for the FP64 sums
             L.call('bsk_pairs_create_f64', ctypes.byref(h), int(mode), int(nshell), len(tri),
                    tri.ctypes.data_as(ip),
                    levels.ctypes.data_as(ip) if levels is not None else None)
@@ -580,9 +584,10 @@ class GridEngine:
     @staticmethod
     def pairs64_nwg(ncell):
         """Workgroups of the FP64 pair kernel: up to four per CU, each with at
-        least eight of its 64-cell chunks (512^3 / 32 bins: 512 workgroups 874 us,
-        768 769, 1024 744)."""
-        return int(max(8, min(1024, ncell // 512 // 8 * 8)))
+        least four of its 64-cell chunks (512^3 / 32 bins: 256 workgroups 1100 us,
+        512 924, 1024 908).  From the cells alone, so that a triangle's sum does
+        not depend on the list."""
+        return int(max(8, min(1024, ncell // 256 // 8 * 8)))
 
     def plain_nchunk(self, ncell=None):
         ncell = self.ncell if ncell is None else ncell
@@ -819,20 +824,80 @@ class GridEngine:
     def grid_info(self, tri, max_bytes=None, stream=None):
         """(N_tri, kbar) for each triangle (i, j, k) of bin indices, FP64.
 
-        The unit and |k| shells are made in FP64 x-slab by x-slab and reduced
-        with the tiled FP64 kernel; N_tri is the rounded sum / S^3 (exact
-        integer), kbar = sum(|k| n n) / S^3 / N_tri (NaN where N_tri == 0).
-        """
+        N_tri is the rounded sum / S^3 (exact integer), kbar = sum(|k| n n) /
+        S^3 / N_tri (NaN where N_tri == 0) over FP64 unit and |k| shells, whose
+        products are summed over the mesh's symmetry wedge with orbit weights
+        (bsk_gridinfo_shells), in x slabs of at most max_bytes (default half of
+        free HBM)."""
         tri = np.asarray(tri, dtype=np.int32).reshape(-1, 3)
         T = len(tri)
         if T == 0:
             return np.zeros(0), np.zeros((0, 3))
         if tri.min() < 0 or tri.max() >= self.nb:
             raise IndexError('triangle bin index out of range')
-        N, nb = self.S, self.nb
         if max_bytes is None:
             free, _ = torch.cuda.mem_get_info(self.device)
             max_bytes = int(free * 0.5)
+        if self.pairs64_supported(2 * self.nb, 1):
+            total = self._gridinfo_wedge(tri, max_bytes, stream)
+        else:
+            total = self._gridinfo_tiled(tri, max_bytes, stream)
+        sums = (total / float(self.ncell)).view(T, 4).cpu().numpy()
+        ntri = np.rint(sums[:, 0])
+        kbar = np.full((T, 3), np.nan)
+        nz = ntri != 0
+        kbar[nz] = sums[nz, 1:4] / ntri[nz, None]
+        return ntri, kbar
+
+    def _gridinfo_slab(self, x0, x1):
+        n, nbytes = ctypes.c_longlong(), L.size_out()
+        L.call('bsk_gridinfo_layout', self._plan, x0, x1, ctypes.byref(n), ctypes.byref(nbytes))
+        return n.value, nbytes.value
+
+    def _gridinfo_wedge(self, tri, max_bytes, stream):
+        """The four sums of each triangle over the S^3 mesh, from the wedge."""
+        T, nb = len(tri), self.nb
+        key = (np.ascontiguousarray(tri).tobytes(), 'gridinfo')
+        plan = self._tri_cache.get(key)
+        if plan is None:
+            with torch.cuda.device(self.device):
+                plan = self._tri_cache[key] = PairPlan(tri, nb, L.MODE_AUTO, gridinfo=True)
+        # x slabs whose shells, weights and intermediates fit max_bytes (one
+        # plane at least)
+        cuts, end = [0], self.S // 2 + 1
+        while cuts[-1] < end:
+            x0, x1 = cuts[-1], end
+            while x1 > x0 + 1:
+                n, nbytes = self._gridinfo_slab(x0, x1)
+                if nbytes + (2 * nb + 1) * 8 * n <= max_bytes:
+                    break
+                x1 = x0 + max(1, (x1 - x0) // 2)
+            cuts.append(x1)
+        s = stream_handle(stream)
+        total = None
+        for x0, x1 in zip(cuts[:-1], cuts[1:]):
+            n, nbytes = self._gridinfo_slab(x0, x1)
+            wk = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+            buf = torch.empty((2 * nb + 1, n), dtype=torch.float64, device=self.device)
+            L.call('bsk_gridinfo_shells', self._plan, x0, x1, L.ptr(buf), n, L.ptr(buf[2 * nb]),
+                   L.ptr(wk), s)
+            # at least four 64-cell chunks per workgroup, at most 256 MB of
+            # partials (2 KB per item and workgroup)
+            nwg = int(max(8, min(512, n // 256, (1 << 17) // plan.nitem) // 8 * 8))
+            size = L.size_out()
+            L.call('bsk_triples_mfma_workspace', plan.handle, nwg, ctypes.byref(size))
+            part = torch.empty(4 * T, dtype=torch.float64, device=self.device)
+            L.call('bsk_triples_f64', plan.handle, None, L.ptr(buf), None, n, n, None, None,
+                   L.ptr(buf[2 * nb]), nwg, 1.0, L.ptr(part),
+                   L.ptr(self.work.get('mfma', size.value)), s)
+            total = part if total is None else total + part
+        return total
+
+    def _gridinfo_tiled(self, tri, max_bytes, stream):
+        """The same sums x slab by x slab of the whole mesh with the tiled FP64
+        kernel, for more shells than the pair kernel holds."""
+        T = len(tri)
+        N, nb = self.S, self.nb
         plane = N * N * 8 * 2 * nb
         xs = int(max(1, min(N, max_bytes // max(plane, 1))))
         while N % xs:
@@ -863,12 +928,7 @@ class GridEngine:
             L.call('bsk_triples_tiled', L.DT_F64, L.ptr(buf), scells, 2 * nb, scells, T,
                    L.ptr(tri_d), 4, nchunk, 1.0, L.ptr(part), L.ptr(wt), s)
             total += part
-        sums = (total / float(self.ncell)).view(T, 4).cpu().numpy()
-        ntri = np.rint(sums[:, 0])
-        kbar = np.full((T, 3), np.nan)
-        nz = ntri != 0
-        kbar[nz] = sums[nz, 1:4] / ntri[nz, None]
-        return ntri, kbar
+        return total
 
     # -------------------------------------------------------- power spectrum
     def power_spectrum(self, dk, stream=None, work=None):

@@ -352,6 +352,22 @@ int bsk_triples_f64(const bsk_pairs* pairs, const double* f_i, const double* f_j
                     const long long* level_off, const long long* level_ncell,
                     const double* weight, int nwg, double scale, double* out_dev, void* work,
                     void* stream);
+/* Grid info over the symmetry wedge.  The unit and |k| shells of N_tri and
+ * the mean wavenumbers depend on |n| alone, so their products are the same at
+ * all cells of an orbit of the cube's symmetries, and a sum over the S^3 mesh
+ * is the sum over the cells S/2 >= x >= y >= z >= 0 weighted by the orbits'
+ * sizes.  bsk_gridinfo_shells makes the FP64 unit shells (rows 0..nbin-1) and
+ * |k| shells (rows nbin..2 nbin-1) of the wedge planes [x0, x1) and the
+ * weights; bsk_gridinfo_layout gives the cells of a row (padded to 64, the
+ * padding weighted 0) and the workspace.  bsk_gridinfo_pairs plans the four
+ * sums of each triangle (i, j, k) for bsk_triples_f64 (out[4t]: n_i n_j n_k,
+ * out[4t + 1 + e]: side e's unit shell replaced by its |k| shell).  Replaces
+ * measure_gridinfo_faster's shells and sums (bskit/main.py:2006-2064). */
+int bsk_gridinfo_layout(const bsk_plan* plan, int x0, int x1, long long* ncell,
+                        size_t* work_bytes);
+int bsk_gridinfo_shells(bsk_plan* plan, int x0, int x1, double* shells, long long shell_stride,
+                        double* weight, void* work, void* stream);
+int bsk_gridinfo_pairs(bsk_pairs** pairs, int nbin, int ntri, const int* tri_host);
 /* out_dev == NULL in bsk_triples_mfma leaves the per-workgroup partials in
  * work; bsk_triples_mfma_reduce then sums them in FP64 into out_dev (the
  * same result as one call with out_dev; it uses the tail of work, after the

@@ -45,7 +45,7 @@ def check(eng, dks, tri, levels, nwg=None):
 
 
 @pytest.mark.parametrize('N,nb,width,nfield,mesh,levels,nwg', [
-    (24, 3, 2, 1, 24, False, None),    # 216 chunks, one tile, lists replicated over the waves
+    (24, 3, 2, 1, 24, False, None),    # 216 chunks, one tile
     (64, 8, 2, 1, None, True, 24),
     (120, 8, 2, 3, None, False, None),  # <ABC>
     (120, 20, 1, 2, None, True, 8),     # <AAB>, a window that starts inside a block
@@ -72,6 +72,17 @@ def test_lists():
     rng = np.random.default_rng(1)
     check(eng, dks, np.concatenate([tri[rng.permutation(len(tri))], tri[:5, ::-1]]), True)
     check(eng, dks, tri[3:4], True)
+
+
+def test_list_independent():
+    """A triangle's sum is the same bits whatever list it is summed with."""
+    eng, dks, tri = setup(128, 17, 2, 1)
+    sh = shells(eng, dks, True)
+    a = eng.triples(sh, tri, path=PATH_PAIRS64).cpu().numpy()
+    rng = np.random.default_rng(5)
+    for pick in (rng.permutation(len(tri))[:40], np.arange(3), [len(tri) - 1]):
+        b = eng.triples(sh, tri[pick][:, [2, 1, 0]], path=PATH_PAIRS64).cpu().numpy()
+        assert np.array_equal(a[pick], b)
 
 
 def test_refusals():
