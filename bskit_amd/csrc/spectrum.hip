@@ -7,13 +7,18 @@
 // of the full spectrum.  By Parseval these equal the cell sums of squared
 // shell fields used by a real-space estimator: sum_x d_b^2 = N^3 S_P,
 // sum_x n_b^2 = N^3 S_N, sum_x (c2r of |k|^(1/2) mask)^2 = N^3 S_K.
-// Grid (nchunk, nbin): each block sums its chunk of the cube for one bin
-// with a fixed-order tree; a second kernel adds the chunks in order (FP64).
+// Grid (nchunk, nbin): each block sums a bin's modes in its chunk of the
+// cube's rows with a fixed-order tree; a second kernel adds the chunks in
+// order (FP64).  A thread takes a row (nx, ny) and only the kz interval the
+// bin holds of it, so all bins together read each mode once: 40 bins at 400^3
+// (17e6 modes retained) 79 us (four lanes per row; one 91), with a test of every
+// mode per bin 1090 us.
 #include "launch.h"
 
 namespace {
 
 constexpr int kT = 256;
+constexpr int kL = 4;  // lanes per row
 
 template <typename T>
 __global__ __launch_bounds__(kT) void k_spectrum(const cplx<T>* __restrict__ dk, Geom g, int N,
@@ -22,22 +27,26 @@ __global__ __launch_bounds__(kT) void k_spectrum(const cplx<T>* __restrict__ dk,
                                                  int nchunk, double* __restrict__ partial) {
   __shared__ double red[3][kT];
   const int b = blockIdx.y, c = blockIdx.x;
-  const long long total = (long long)g.MX * g.MY * g.MZ;
-  const long long e0 = total * c / nchunk, e1 = total * (c + 1) / nchunk;
+  const int rows = g.MX * g.MY;
+  const int r0 = (int)((long long)rows * c / nchunk), r1 = (int)((long long)rows * (c + 1) / nchunk);
   const int lo = n2lo[b], hi = n2hi[b];
   double sp = 0.0, sn = 0.0, sk = 0.0;
-  for (long long e = e0 + threadIdx.x; e < e1; e += kT) {
-    const int kz = (int)(e % g.MZ);
-    const long long r = e / g.MZ;
-    const int rx = (int)(r % g.MX), ry = (int)(r / g.MX);
-    const int nx = g.nlo + rx, ny = g.nlo + ry;
-    const int n2 = nx * nx + ny * ny + kz * kz;
-    if (n2 < lo || n2 > hi) continue;
-    const double w = (kz == 0 || 2 * kz == N) ? 1.0 : 2.0;
-    const cplx<T> v = dk[e];
-    sp += w * ((double)v.x * v.x + (double)v.y * v.y);
-    sn += w;
-    sk += w * kf * sqrt((double)n2);
+  const int l = threadIdx.x & (kL - 1);
+  for (int r = r0 + threadIdx.x / kL; r < r1; r += kT / kL) {
+    const int ry = r / g.MX, nx = g.nlo + r - ry * g.MX, ny = g.nlo + ry;
+    const int r2 = nx * nx + ny * ny;
+    if (r2 > hi) continue;
+    const int k1 = min(isqrt_floor(hi - r2), g.MZ - 1);
+    int k0 = lo > r2 ? isqrt_floor(lo - r2) : 0;
+    if (k0 * k0 + r2 < lo) ++k0;
+    const cplx<T>* row = dk + (long long)r * g.MZ;
+    for (int kz = k0 + l; kz <= k1; kz += kL) {
+      const double w = (kz == 0 || 2 * kz == N) ? 1.0 : 2.0;
+      const cplx<T> v = row[kz];
+      sp += w * ((double)v.x * v.x + (double)v.y * v.y);
+      sn += w;
+      sk += w * kf * sqrt((double)(r2 + kz * kz));
+    }
   }
   red[0][threadIdx.x] = sp;
   red[1][threadIdx.x] = sn;
