@@ -32,6 +32,8 @@ _dbl_p = ctypes.POINTER(ctypes.c_double)
 _SIGS = {
     'bsk_version': [],
     'bsk_last_error': [],
+    'bsk_closed_triangles': [_c_int, _dbl_p, _dbl_p, _c_int, ctypes.POINTER(_c_ll),
+                             ctypes.POINTER(_c_ll)],
     'bsk_shell_thresholds': [_c_int, _c_double, _c_int, _dbl_p, _dbl_p, _int_p, _int_p],
     'bsk_plan_create': [ctypes.POINTER(_vp), _c_int, _c_double, _c_int, _dbl_p, _dbl_p],
     'bsk_plan_destroy': [_vp],
@@ -141,6 +143,19 @@ def lib():
                                   % (LIB_PATH, h.bsk_version(), ABI_VERSION))
             _lib = h
     return _lib
+
+
+def built():
+    """Whether the library is there to load (host-only helpers have numpy twins)."""
+    return _lib is not None or os.path.exists(LIB_PATH)
+
+
+def dbl_ptr(a):
+    return a.ctypes.data_as(_dbl_p)
+
+
+def ll_ptr(a):
+    return a.ctypes.data_as(ctypes.POINTER(_c_ll))
 
 
 def exported_symbols():

@@ -323,6 +323,30 @@ const char* bsk_last_error(void) { return g_err; }
 
 int bsk_version(void) { return BSK_ABI_VERSION; }
 
+int bsk_closed_triangles(int nbin, const double* lo, const double* hi, int num_fields,
+                         long long* count, long long* out) {
+  if (nbin < 0 || (nbin && (!lo || !hi)) || !count) {
+    bsk_set_error("bsk_closed_triangles: invalid argument");
+    return BSK_EINVAL;
+  }
+  long long n = 0;
+  for (int i = 0; i < nbin; ++i)
+    for (int j = 0; j < (num_fields <= 2 ? i + 1 : nbin); ++j) {
+      const double hij = hi[i] + hi[j];
+      for (int k = 0; k < (num_fields == 1 ? j + 1 : nbin); ++k) {
+        if (!(hij >= lo[k] && hi[i] + hi[k] >= lo[j] && hi[j] + hi[k] >= lo[i])) continue;
+        if (out) {
+          out[3 * n] = i;
+          out[3 * n + 1] = j;
+          out[3 * n + 2] = k;
+        }
+        ++n;
+      }
+    }
+  *count = n;
+  return BSK_OK;
+}
+
 int bsk_shell_thresholds(int nmesh, double box_size, int nbin, const double* k_low,
                          const double* k_high, int* n2lo, int* n2hi) {
   if (nmesh <= 0 || box_size <= 0 || nbin < 0 || (nbin && (!k_low || !k_high || !n2lo || !n2hi))) {

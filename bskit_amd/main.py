@@ -36,7 +36,7 @@ from . import _lib as L
 from . import io as bio
 from .bins import (generate_bin_edge_list, generate_equilateral_triangle_bin_list,
                    generate_isosceles_triangle_bin_list, generate_squeezed_triangle_bin_list,
-                   generate_triangle_bin_list, geometric_k_mean)
+                   generate_triangle_bin_list, geometric_k_mean, triangle_bins)
 from .engine import GridEngine, require_device
 from .mesh import ArrayMesh, MeshSource, ParticleMesh, cast_source
 
@@ -170,8 +170,7 @@ class FFTBispectrum:
             if triangle_type == 'all':
                 kw = dict(kmin=kmin, kmax=kmax, dk=dk, dmu=dmu, mu_min=mu_min, mu_max=mu_max,
                           num_fields=self.num_fields, **args)
-                self.k_edges = generate_triangle_bin_list(**kw)
-                self.k_indices = generate_triangle_bin_list(return_indices=True, **kw)
+                self.k_edges, self.k_indices = triangle_bins(**kw)
             elif triangle_type == 'equilateral':
                 self.k_edges = generate_equilateral_triangle_bin_list(kmin, kmax, dk, **args)
                 self.k_indices = generate_equilateral_triangle_bin_list(kmin, kmax, dk, **args,
@@ -345,12 +344,14 @@ class FFTBispectrum:
         out = eng.triples(sets, tri, path=path, scale=factor / float(eng.ncell))
         return out.cpu().numpy()
 
-    def _append_b(self, index, edges, kmean, B, ntri):
+    def _append_b(self, index, edges, kmean, B, ntri, own=('index', 'B')):
+        """own: the arrays made for this call (stored as they are; the others
+        are copied, being views of k_edges or kept by the engine)."""
         new = {'index': np.asarray(index), 'k_edge': np.asarray(edges).reshape(-1, 6),
                'k_mean': np.asarray(kmean, dtype=np.float64).reshape(-1, 3),
                'B': np.asarray(B, dtype=np.float64), 'N_tri': np.asarray(ntri, dtype=np.float64)}
         if self.b is None:
-            self.b = {k: v.copy() for k, v in new.items()}
+            self.b = {k: v if k in own else v.copy() for k, v in new.items()}
         else:
             for k, v in new.items():
                 self.b[k] = np.append(self.b[k], v, axis=0)
@@ -424,7 +425,8 @@ class FFTBispectrum:
                 print('FFT Bk: %d %d %g' % (t, index[t], B[t]))
         if out_file is not None and T:
             bio.append_rows(out_file, bio.FAST_B, index, edges, B=B)
-        return self._append_b(index, edges, np.zeros((T, 3)), B, np.zeros(T))
+        return self._append_b(index, edges, np.zeros((T, 3)), B, np.zeros(T),
+                              own=('index', 'B', 'k_mean', 'N_tri'))
 
     def measure_gridinfo_faster(self, imin=None, imax=None, kmeas_min=None, kmeas_max=None,
                                 out_file=None, verbose=0):

@@ -67,6 +67,14 @@ typedef struct bsk_plan bsk_plan;
 const char* bsk_last_error(void);
 int bsk_version(void);
 
+/* Index triples (i, j, k) of bins [lo, hi] that can close a triangle (every
+ * side's lower edge at most the sum of the other two upper edges), host arrays,
+ * in lexicographic order: i >= j >= k for one field, i >= j for two, all for
+ * three.  *count = their number; out (3 per triple) may be NULL.  Replaces the
+ * filter of generate_triangle_bin_list (bskit/main.py:1331-1340). */
+int bsk_closed_triangles(int nbin, const double* lo, const double* hi, int num_fields,
+                         long long* count, long long* out);
+
 /* Integer |n|^2 limits of the closed shells [k_low[b], k_high[b]].
  * Replaces the float mask predicate (kk<=kmax)&(kk>=kmin) of
  * bskit/main.py:264-268, :314-320, :1850-1852. */
