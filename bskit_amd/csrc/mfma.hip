@@ -49,7 +49,6 @@ BSK_DEV float bf_sum_hi(uint32_t h, uint32_t l, bf16x2 one_hi) {
 
 constexpr int kW = kPairWaves;   // waves per workgroup
 constexpr int kNT = 64 * kW;
-constexpr int kCK = kPairChunk;  // cells per staged chunk
 // LDS layout (strides chosen by measured ds_read_b128 throughput on gfx950):
 //  * FP32 pair-side rows of 136 floats (544 B), cells in natural order; in a
 //    K step lane group g reads cells 4g..4g+3 and 16+4g..16+4g+3, the pattern
@@ -58,10 +57,17 @@ constexpr int kCK = kPairChunk;  // cells per staged chunk
 //    permuted so that lane group g finds the same eight cells contiguous at
 //    8g: cell 4g+e at 8g+e and cell 16+4g+e at 8g+4+e (e < 4).  The MFMA K
 //    order is then the same permutation on both operands.
-constexpr int kLDF = kCK + 8;    // FP32 row stride (floats)
-constexpr int kLDH = kCK + 16;   // bf16 row stride (elements)
-constexpr int kSEGS = kCK / 8;   // 16-byte segments per row and plane
-constexpr int kKSTEPS = kCK / 32;
+// A chunk is CK = kPairChunk cells, or half of it where the staged shells would
+// leave one workgroup per CU (above about 60 shells): the same K steps in the
+// same order, so the same bits.  1024^3 / 80 bins (99 KB staged by whole chunks): the
+// E and O segments 2013 -> 1372 us each.
+template <int CK>
+struct Chunk {
+  static constexpr int LDF = CK + 8;    // FP32 row stride (floats)
+  static constexpr int LDH = CK + 16;   // bf16 row stride (elements)
+  static constexpr int SEGS = CK / 8;   // 16-byte segments per row and plane
+  static constexpr int KSTEPS = CK / 32;
+};
 
 // Per-thread share of one staged shell set: PV 16-byte segments of the hi
 // and lo planes, loaded one chunk ahead and stored to LDS afterwards.
@@ -70,9 +76,10 @@ struct Pref {
   uint4 h[PV], l[PV];
 };
 
-template <int PV>
+template <int CK, int PV>
 BSK_DEV void fetch(Pref<PV>& p, const uint16_t* __restrict__ gh, const uint16_t* __restrict__ gl,
                    long long stride, int n, long long cbase) {
+  constexpr int kSEGS = Chunk<CK>::SEGS;
 #pragma unroll
   for (int k = 0; k < PV; ++k) {
     const int v = threadIdx.x + k * kNT;
@@ -88,9 +95,10 @@ BSK_DEV void fetch(Pref<PV>& p, const uint16_t* __restrict__ gh, const uint16_t*
 // The same loads issued by every thread (threads past the staged rows
 // re-read row 0), so a wave always has the same number of loads in flight
 // and a wait for an older chunk's loads can leave a newer chunk's pending.
-template <int PV>
+template <int CK, int PV>
 BSK_DEV void fetch_all(Pref<PV>& p, const uint16_t* __restrict__ gh,
                        const uint16_t* __restrict__ gl, long long stride, int n, long long cbase) {
+  constexpr int kSEGS = Chunk<CK>::SEGS;
 #pragma unroll
   for (int k = 0; k < PV; ++k) {
     int v = threadIdx.x + k * kNT;
@@ -104,8 +112,9 @@ BSK_DEV void fetch_all(Pref<PV>& p, const uint16_t* __restrict__ gh,
 
 // FP32 values d = hi + lo to f (if non-null) and raw planes to h/l (if
 // non-null) for rows < n.
-template <int PV>
+template <int CK, int PV>
 BSK_DEV void put(const Pref<PV>& p, int n, float* f, uint16_t* h, uint16_t* l) {
+  constexpr int kSEGS = Chunk<CK>::SEGS, kLDF = Chunk<CK>::LDF, kLDH = Chunk<CK>::LDH;
   const bf16x2 olo = bf16_pair_bits(kBf16OneLo), ohi = bf16_pair_bits(kBf16OneHi);
 #pragma unroll
   for (int k = 0; k < PV; ++k) {
@@ -152,8 +161,10 @@ constexpr int pair_occupancy() {
 // D2 (one field, one prefetch segment per thread): two chunks in flight
 // per workgroup instead of one, for segments whose few items leave the
 // staging loads' latency exposed (replicated wave lists).
-template <int NI, int PV, int SETS, bool D2>
+template <int NI, int PV, int SETS, bool D2, int CK>
 __global__ __launch_bounds__(kNT, (pair_occupancy<NI, PV, SETS, D2>())) void k_triple_pairs(PairArgs a) {
+  constexpr int kCK = CK, kLDF = Chunk<CK>::LDF, kLDH = Chunk<CK>::LDH,
+                kKSTEPS = Chunk<CK>::KSTEPS;
   static_assert(!D2 || (SETS == 1 && PV == 1), "two-chunk prefetch: one field, one segment");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int n0 = a.nsh[0], n1 = a.nsh[1], n2 = a.nsh[2];
@@ -202,9 +213,9 @@ __global__ __launch_bounds__(kNT, (pair_occupancy<NI, PV, SETS, D2>())) void k_t
   State<NI> st;
   init(st);
 
-  const long long nch = a.ncell / kCK;
-  const long long ch0 = nch * lw / a.nwg;
-  const long long ch1 = nch * (lw + 1) / a.nwg;
+  const long long nch = a.ncell / kPairChunk;  // the same cell ranges for either chunk
+  const long long ch0 = nch * lw / a.nwg * (kPairChunk / CK);
+  const long long ch1 = nch * (lw + 1) / a.nwg * (kPairChunk / CK);
   auto ksteps = [&]() {
 #pragma unroll  // constant LDS offsets per K step
     for (int ks = 0; ks < kKSTEPS; ++ks)
@@ -219,24 +230,24 @@ __global__ __launch_bounds__(kNT, (pair_occupancy<NI, PV, SETS, D2>())) void k_t
     if (ch0 < ch1) {
       const long long last = ch1 - 1;
       Pref<PV> qa, qb;
-      fetch_all(qa, a.hi[0], a.lo[0], a.stride, n0, ch0 * kCK);
-      fetch_all(qb, a.hi[0], a.lo[0], a.stride, n0, (ch0 + 1 < last ? ch0 + 1 : last) * kCK);
+      fetch_all<CK>(qa, a.hi[0], a.lo[0], a.stride, n0, ch0 * kCK);
+      fetch_all<CK>(qb, a.hi[0], a.lo[0], a.stride, n0, (ch0 + 1 < last ? ch0 + 1 : last) * kCK);
       long long ch = ch0;
       for (; ch + 1 < ch1; ch += 2) {  // chunk pairs
         __syncthreads();  // every wave is done with the previous chunk
-        put(qa, n0, fA, hKs, lKs);
+        put<CK>(qa, n0, fA, hKs, lKs);
         __syncthreads();
-        fetch_all(qa, a.hi[0], a.lo[0], a.stride, n0, (ch + 2 < last ? ch + 2 : last) * kCK);
+        fetch_all<CK>(qa, a.hi[0], a.lo[0], a.stride, n0, (ch + 2 < last ? ch + 2 : last) * kCK);
         ksteps();
         __syncthreads();
-        put(qb, n0, fA, hKs, lKs);
+        put<CK>(qb, n0, fA, hKs, lKs);
         __syncthreads();
-        fetch_all(qb, a.hi[0], a.lo[0], a.stride, n0, (ch + 3 < last ? ch + 3 : last) * kCK);
+        fetch_all<CK>(qb, a.hi[0], a.lo[0], a.stride, n0, (ch + 3 < last ? ch + 3 : last) * kCK);
         ksteps();
       }
       if (ch < ch1) {  // odd count: the last chunk
         __syncthreads();
-        put(qa, n0, fA, hKs, lKs);
+        put<CK>(qa, n0, fA, hKs, lKs);
         __syncthreads();
         ksteps();
       }
@@ -244,21 +255,21 @@ __global__ __launch_bounds__(kNT, (pair_occupancy<NI, PV, SETS, D2>())) void k_t
   } else {
     Pref<PV> p0, p1, p2;
     if (ch0 < ch1) {
-      fetch(p0, a.hi[0], a.lo[0], a.stride, n0, ch0 * kCK);
-      if (SETS == 3) fetch(p1, a.hi[1], a.lo[1], a.stride, n1, ch0 * kCK);
-      if (SETS >= 2) fetch(p2, a.hi[2], a.lo[2], a.stride, n2, ch0 * kCK);
+      fetch<CK>(p0, a.hi[0], a.lo[0], a.stride, n0, ch0 * kCK);
+      if (SETS == 3) fetch<CK>(p1, a.hi[1], a.lo[1], a.stride, n1, ch0 * kCK);
+      if (SETS >= 2) fetch<CK>(p2, a.hi[2], a.lo[2], a.stride, n2, ch0 * kCK);
     }
     for (long long ch = ch0; ch < ch1; ++ch) {
       __syncthreads();  // every wave is done with the previous chunk
-      put(p0, n0, fA, SETS == 1 ? hKs : nullptr, SETS == 1 ? lKs : nullptr);
-      if (SETS == 3) put(p1, n1, fB, nullptr, nullptr);
-      if (SETS >= 2) put(p2, n2, nullptr, hKs, lKs);
+      put<CK>(p0, n0, fA, SETS == 1 ? hKs : nullptr, SETS == 1 ? lKs : nullptr);
+      if (SETS == 3) put<CK>(p1, n1, fB, nullptr, nullptr);
+      if (SETS >= 2) put<CK>(p2, n2, nullptr, hKs, lKs);
       __syncthreads();
       if (ch + 1 < ch1) {  // next chunk's HBM loads overlap this chunk's math
         const long long cb = (ch + 1) * kCK;
-        fetch(p0, a.hi[0], a.lo[0], a.stride, n0, cb);
-        if (SETS == 3) fetch(p1, a.hi[1], a.lo[1], a.stride, n1, cb);
-        if (SETS >= 2) fetch(p2, a.hi[2], a.lo[2], a.stride, n2, cb);
+        fetch<CK>(p0, a.hi[0], a.lo[0], a.stride, n0, cb);
+        if (SETS == 3) fetch<CK>(p1, a.hi[1], a.lo[1], a.stride, n1, cb);
+        if (SETS >= 2) fetch<CK>(p2, a.hi[2], a.lo[2], a.stride, n2, cb);
       }
       ksteps();
     }
@@ -334,9 +345,9 @@ __global__ __launch_bounds__(256) void k_reduce_tri(const double* __restrict__ s
   out[t] = s * scale * f;
 }
 
-template <int NI, int PV, int SETS, bool D2>
+template <int NI, int PV, int SETS, bool D2, int CK>
 int launch_pairs(const PairArgs& a, size_t lds, hipStream_t s) {
-  auto fn = k_triple_pairs<NI, PV, SETS, D2>;
+  auto fn = k_triple_pairs<NI, PV, SETS, D2, CK>;
   // once per instance (not per launch: keeps launches capturable and cheap)
   static const hipError_t attr = hipFuncSetAttribute(
       (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -348,22 +359,22 @@ int launch_pairs(const PairArgs& a, size_t lds, hipStream_t s) {
 
 // Replicated wave lists (few items per workgroup) with one field and one
 // prefetch segment per thread run the two-chunk prefetch.
-template <int NI, int PV, int SETS>
+template <int NI, int PV, int SETS, int CK>
 int launch_d2(const PairArgs& a, size_t lds, hipStream_t s) {
-  if constexpr (SETS == 1 && PV == 1 && NI <= 4 && NI != 2)  // NI = 2: no registers to spare
-    if (a.rep > 1) return launch_pairs<NI, PV, SETS, true>(a, lds, s);
-  return launch_pairs<NI, PV, SETS, false>(a, lds, s);
+  if constexpr (SETS == 1 && PV == 1 && NI <= 4 && NI != 2 && CK == kPairChunk)  // NI = 2: no registers to spare
+    if (a.rep > 1) return launch_pairs<NI, PV, SETS, true, CK>(a, lds, s);
+  return launch_pairs<NI, PV, SETS, false, CK>(a, lds, s);
 }
 
-template <int PV, int SETS>
+template <int PV, int SETS, int CK>
 int launch_ni(const PairArgs& a, int ni, size_t lds, hipStream_t s) {
   switch (ni) {
-    case 1: return launch_d2<1, PV, SETS>(a, lds, s);
-    case 2: return launch_d2<2, PV, SETS>(a, lds, s);
-    case 3: return launch_d2<3, PV, SETS>(a, lds, s);
-    case 4: return launch_d2<4, PV, SETS>(a, lds, s);
-    case 6: return launch_pairs<6, PV, SETS, false>(a, lds, s);
-    case 8: return launch_pairs<8, PV, SETS, false>(a, lds, s);
+    case 1: return launch_d2<1, PV, SETS, CK>(a, lds, s);
+    case 2: return launch_d2<2, PV, SETS, CK>(a, lds, s);
+    case 3: return launch_d2<3, PV, SETS, CK>(a, lds, s);
+    case 4: return launch_d2<4, PV, SETS, CK>(a, lds, s);
+    case 6: return launch_pairs<6, PV, SETS, false, CK>(a, lds, s);
+    case 8: return launch_pairs<8, PV, SETS, false, CK>(a, lds, s);
     default:
       bsk_set_error("mfma triple: %d items per wave not compiled", ni);
       return BSK_EUNSUPPORTED;
@@ -371,15 +382,22 @@ int launch_ni(const PairArgs& a, int ni, size_t lds, hipStream_t s) {
 }
 
 template <int SETS>
-int launch_pv(const PairArgs& a, int ni, int pv, size_t lds, hipStream_t s) {
+int launch_pv(const PairArgs& a, int ni, int pv, bool half, size_t lds, hipStream_t s) {
+  if (half) return launch_ni<2, SETS, kPairChunk / 2>(a, ni, lds, s);
   switch (pv) {
-    case 1: return launch_ni<1, SETS>(a, ni, lds, s);
-    case 2: return launch_ni<2, SETS>(a, ni, lds, s);
-    case 4: return launch_ni<4, SETS>(a, ni, lds, s);
+    case 1: return launch_ni<1, SETS, kPairChunk>(a, ni, lds, s);
+    case 2: return launch_ni<2, SETS, kPairChunk>(a, ni, lds, s);
+    case 4: return launch_ni<4, SETS, kPairChunk>(a, ni, lds, s);
     default:
       bsk_set_error("mfma triple: %d prefetch segments per thread not compiled", pv);
       return BSK_EUNSUPPORTED;
   }
+}
+
+template <int CK>
+size_t lds_bytes(int sets, const int nsh[3], int nkb) {
+  const size_t frows = (size_t)(nsh[0] + 1) + (sets == 3 ? (size_t)(nsh[1] + 1) : 0);
+  return frows * Chunk<CK>::LDF * 4 + (size_t)2 * 16 * nkb * Chunk<CK>::LDH * 2;
 }
 
 }  // namespace
@@ -399,18 +417,17 @@ int bsk_pair_item_cap(int sets, int nshell) {
 }
 
 int bsk_pair_prefetch(int nshell) {
-  const int pv = (nshell * kSEGS + kNT - 1) / kNT;
+  const int pv = (nshell * Chunk<kPairChunk>::SEGS + kNT - 1) / kNT;
   return pv <= 1 ? 1 : (pv <= 2 ? 2 : (pv <= 4 ? 4 : 0));
 }
 
 size_t bsk_pair_lds_bytes(int sets, const int nsh[3], int nkb) {
-  const size_t frows = (size_t)(nsh[0] + 1) + (sets == 3 ? (size_t)(nsh[1] + 1) : 0);
-  return frows * kLDF * 4 + (size_t)2 * 16 * nkb * kLDH * 2;
+  return lds_bytes<kPairChunk>(sets, nsh, nkb);
 }
 
 int bsk_triple_pairs_launch(const PairArgs& a, int sets, int ni, hipStream_t s) {
-  if (a.ncell % kCK) {
-    bsk_set_error("mfma triple: cell count %lld not a multiple of %d", a.ncell, kCK);
+  if (a.ncell % kPairChunk) {
+    bsk_set_error("mfma triple: cell count %lld not a multiple of %d", a.ncell, kPairChunk);
     return BSK_EINVAL;
   }
   if (a.nsh[0] < 1 || a.nsh[1] < 1 || a.nsh[2] < 1) {
@@ -432,17 +449,22 @@ int bsk_triple_pairs_launch(const PairArgs& a, int sets, int ni, hipStream_t s) 
     bsk_set_error("mfma triple: %d replicas (1, 2 or 4)", a.rep);
     return BSK_EINVAL;
   }
+  // half chunks where whole ones leave one workgroup per CU (replicated lists
+  // split the four K steps of a whole one)
+  const bool half = a.rep == 1 && bsk_pair_lds_bytes(sets, a.nsh, a.nkb) > 80 * 1024 && nmax <= 128;
   // LDS: the staging, and the replicas' tiles (FP64) at the end
-  const size_t lds = std::max(bsk_pair_lds_bytes(sets, a.nsh, a.nkb),
-                              (size_t)(a.rep - 1) * (kW / a.rep) * ni * 256 * 8);
+  const size_t lds =
+      half ? lds_bytes<kPairChunk / 2>(sets, a.nsh, a.nkb)
+           : std::max(bsk_pair_lds_bytes(sets, a.nsh, a.nkb),
+                      (size_t)(a.rep - 1) * (kW / a.rep) * ni * 256 * 8);
   if (!pv || lds > 160 * 1024) {
     bsk_set_error("mfma triple: %d shells exceed the kernel's staging (LDS %zu bytes)", nmax,
                   lds);
     return BSK_EUNSUPPORTED;
   }
-  if (sets == 1) return launch_pv<1>(a, ni, pv, lds, s);
-  if (sets == 2) return launch_pv<2>(a, ni, pv, lds, s);
-  if (sets == 3) return launch_pv<3>(a, ni, pv, lds, s);
+  if (sets == 1) return launch_pv<1>(a, ni, pv, half, lds, s);
+  if (sets == 2) return launch_pv<2>(a, ni, pv, half, lds, s);
+  if (sets == 3) return launch_pv<3>(a, ni, pv, half, lds, s);
   bsk_set_error("mfma triple: sets must be 1, 2 or 3");
   return BSK_EINVAL;
 }
