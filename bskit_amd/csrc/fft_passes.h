@@ -559,9 +559,15 @@ __global__ __launch_bounds__(W) void k_inv_z(const cplx<T>* __restrict__ in, voi
   constexpr int LD = pencil_ld<NH>();
   constexpr int KH = NH / 2 + 1;  // k = 0..NH/2 (each with its mirror NH - k)
   // lanes per row for the pairs: at most the workgroup, each lane then
-  // taking KS pairs of its row (KS = 1 unless NH/2 + 1 > W)
-  constexpr int KQ = pow2_at_least(KH) < W ? pow2_at_least(KH) : W;
-  constexpr int KS = (KH + KQ - 1) / KQ, RK = W / KQ, NPK = P / RK;
+  // taking KS pairs of its row (KS = 1 unless NH/2 + 1 > W).  Where NH is a
+  // power of two, NH/2 + 1 pairs would leave half the lanes idle: MID, the
+  // self-mirrored k = NH/2 of every row is a lane's extra item instead
+  // (80 shells of 256^3: 1.90 -> 1.57 ms, 7.5 GB at 4.8 TB/s; the HBM traffic
+  // bounds it, as on the other meshes).
+  constexpr bool MID = (NH & (NH - 1)) == 0 && P <= W && NH / 2 <= W;
+  constexpr int KL = MID ? NH / 2 : KH;  // pairs of the main loop
+  constexpr int KQ = pow2_at_least(KL) < W ? pow2_at_least(KL) : W;
+  constexpr int KS = (KL + KQ - 1) / KQ, RK = W / KQ, NPK = P / RK;
   constexpr int QQ = pow2_at_least(NH / 4) > W / P ? pow2_at_least(NH / 4) : W / P;
   constexpr int RQ = W / QQ, NPQ = P / RQ;
   using Lay = ShellLevels<NH>;
@@ -578,15 +584,22 @@ __global__ __launch_bounds__(W) void k_inv_z(const cplx<T>* __restrict__ in, voi
   const int tid = threadIdx.x;
   stage_in<T, TWS, W>([&](int i) { return twg[2 * i]; }, [&](int i, cplx<T> v) { tw[i] = v; });
   __syncthreads();
-  const long long row0 = (long long)blockIdx.x * P;
   const long long bl = blockIdx.y;
+  const int pm = parts ? parts[bl] : 0xf;  // parts written of this shell (level layout)
+  // Pencil p transforms row row0 + prow(p), p < np.  P rows per workgroup, or,
+  // for a shell whose parts hold only E and O, the P rows with x + y even of
+  // GP rows (x + y odd feeds neither; y = row mod 2 as N is even)
+  constexpr int GP = (N >= 2 * P || N == P) ? 2 * P : P;
+  const bool gather = lv && !(pm & 0x9) && N >= P;
+  const int rows = gather ? GP : P;
+  const long long row0 = (long long)blockIdx.x * rows;
+  if (row0 >= nrows) return;                        // uniform
   const int mzb = shell_mz(MZ, n2hi[shell0 + bl]);  // kz from mzb on are zero
   const cplx<T>* src = in + (bl * nrows + row0) * MZP;
   const int esz = out_esize<T>(fmt);
   // uniform base of the level layout: this shell's row
   char* const shi = static_cast<char*>(out) + bl * shell_stride * esz;
   char* const slo = out_lo ? static_cast<char*>(out_lo) + bl * shell_stride * esz : nullptr;
-  const int pm = parts ? parts[bl] : 0xf;  // parts written of this shell (level layout)
   if (lv && blockIdx.x == 0)  // zero padding of the parts written
 #pragma unroll
     for (int part = 0; part < 4; ++part) {
@@ -595,13 +608,9 @@ __global__ __launch_bounds__(W) void k_inv_z(const cplx<T>* __restrict__ in, voi
       for (long long e = Lay::OFF[part] + Lay::CNT[part] + tid; e < end; e += W)
         store_zero<T>(fmt, shi, slo, (unsigned)e);
     }
-  const int nr = (int)(nrows - row0 < P ? nrows - row0 : P);
-  // Pencil p transforms row row0 + prow(p), p < np.  All nr rows, or, for a
-  // shell whose parts hold only E and O, the rows with x + y even (x + y odd
-  // feeds neither; y = row mod 2 as N is even): n1 of them in the x plane of
-  // row0 from r1, the rest in the next plane from r2 (at most one plane
-  // boundary per workgroup as N >= P), gathered into the first pencils.
-  const bool gather = lv && !(pm & 0x9) && N >= P;
+  const int nr = (int)(nrows - row0 < rows ? nrows - row0 : rows);
+  // gather: n1 of the rows in the x plane of row0 from r1, the rest in the next
+  // plane from r2 (at most one plane boundary among GP rows)
   int np = nr, n1 = nr, r1 = 0, r2 = 0, step = 1;
   if (gather) {
     const long long x0 = row0 / N, b = (x0 + 1) * N, end = row0 + nr;
@@ -622,11 +631,16 @@ __global__ __launch_bounds__(W) void k_inv_z(const cplx<T>* __restrict__ in, voi
   // row: make that explicit so the row index math runs in scalar registers
   const int r0 = KQ >= 64 ? __builtin_amdgcn_readfirstlane(tid / KQ) : tid / KQ;
   constexpr int B = NPK < 8 ? NPK : 8;
+  cplx<T> xm = {(T)0, (T)0};
+  if (MID && tid < np && NH / 2 < mzb) xm = get_u32(src, (unsigned)(prow(tid) * MZP + NH / 2));
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     const int k = (tid & (KQ - 1)) + ks * KQ, j = NH - k;
-    const bool kact = k < KH;
-    const cplx<T> wk = kact ? cconj(twg[k]) : cplx<T>{(T)0, (T)0};  // exp(+2 pi i k / N)
+    const bool kact = k < KL;
+    // exp(+2 pi i k / N), the sign of its sine applied here (folded into the
+    // products it would round them in another order)
+    cplx<T> wk = kact ? cconj(twg[k]) : cplx<T>{(T)0, (T)0};
+    asm("" : "+v"(wk.y));
 #pragma unroll
     for (int q0 = 0; q0 < NPK; q0 += B) {
       cplx<T> xk[B], xj[B];
@@ -644,13 +658,13 @@ __global__ __launch_bounds__(W) void k_inv_z(const cplx<T>* __restrict__ in, voi
           c2r_pair<T>(buf + (r0 + (q0 + q) * RK) * LD, k, NH, xk[q], xj[q], wk);
     }
   }
+  if (MID && tid < P) {
+    cplx<T> wk = cconj(twg[NH / 2]);
+    asm("" : "+v"(wk.y));
+    c2r_pair<T>(buf + tid * LD, NH / 2, NH, xm, xm, wk);
+  }
   __syncthreads();
-  if (gather)
-    fft_lds_n<T, NH, true, P, W, LD, NH>(
-        buf, tw, np, div_magic(np), tid,
-        typename Plan<NH, V>::seq{});
-  else
-    fft_lds<T, NH, true, P, W, LD, NH>(buf, tw, typename Plan<NH, V>::seq{});
+  fft_lds<T, NH, true, P, W, LD, NH>(buf, tw, typename Plan<NH, V>::seq{});
   // four complex values (eight reals, z = 8q .. 8q + 7) per lane and store:
   // in the level layout the four even z and the four odd z are each four
   // consecutive cells of one part
