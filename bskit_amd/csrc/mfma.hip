@@ -13,7 +13,8 @@
 //
 // Workgroup structure (kPairWaves waves, one code path):
 //  * the workgroup owns a contiguous range of CK-cell chunks; per chunk the
-//    hi/lo planes of every shell of each role set are read from HBM once
+//    hi/lo planes of every shell of each role set (of a list in several
+//    passes: those its pass reads) are read from HBM once
 //    (coalesced, prefetched into registers one chunk ahead) and stored in
 //    LDS as FP32 d = hi + lo (pair sides) and as raw bf16 planes (third
 //    side); one zero FP32 row per pair set serves padding rows;
@@ -76,9 +77,35 @@ struct Pref {
   uint4 h[PV], l[PV];
 };
 
+// The rows a thread stages (-1: none; bit 16: the row is a third side of the
+// workgroup's items), pair sides first: rows below nf in that order.  A pass of
+// a long list forms pairs of about half of the staged shells and needs most,
+// not all, of their third-side blocks; LDS writes run at a quarter of the rate
+// of its 16-B reads, so what no item reads is neither loaded nor written.
+// 1024^3 / 80 bins: E (10 passes) and O (6) 1829 and 1009 -> 1762 and 939 us, C0
+// minus E (2) 943 -> 840.
+template <int PV>
+struct RowSet {
+  int r[PV], nf;
+};
+
 template <int CK, int PV>
-BSK_DEV void fetch(Pref<PV>& p, const uint16_t* __restrict__ gh, const uint16_t* __restrict__ gl,
-                   long long stride, int n, long long cbase) {
+BSK_DEV void fetch(Pref<PV>& p, const RowSet<PV>& q, const uint16_t* __restrict__ gh,
+                   const uint16_t* __restrict__ gl, long long stride, long long cbase) {
+  const int sg = threadIdx.x % Chunk<CK>::SEGS;
+#pragma unroll
+  for (int k = 0; k < PV; ++k)
+    if (q.r[k] >= 0) {
+      const long long g = (long long)(q.r[k] & 0xffff) * stride + cbase + sg * 8;
+      p.h[k] = *reinterpret_cast<const uint4*>(gh + g);
+      p.l[k] = *reinterpret_cast<const uint4*>(gl + g);
+    }
+}
+
+// Every row below n.
+template <int CK, int PV>
+BSK_DEV void fetch(Pref<PV>& p, int n, const uint16_t* __restrict__ gh,
+                   const uint16_t* __restrict__ gl, long long stride, long long cbase) {
   constexpr int kSEGS = Chunk<CK>::SEGS;
 #pragma unroll
   for (int k = 0; k < PV; ++k) {
@@ -92,7 +119,7 @@ BSK_DEV void fetch(Pref<PV>& p, const uint16_t* __restrict__ gh, const uint16_t*
   }
 }
 
-// The same loads issued by every thread (threads past the staged rows
+// Loads of every staged row issued by every thread (threads past them
 // re-read row 0), so a wave always has the same number of loads in flight
 // and a wait for an older chunk's loads can leave a newer chunk's pending.
 template <int CK, int PV>
@@ -110,35 +137,52 @@ BSK_DEV void fetch_all(Pref<PV>& p, const uint16_t* __restrict__ gh,
   }
 }
 
-// FP32 values d = hi + lo to f (if non-null) and raw planes to h/l (if
-// non-null) for rows < n.
+// One segment of a row: its FP32 values d = hi + lo to f, its raw planes to
+// h / l (each if non-null).
+template <int CK>
+BSK_DEV void put_segment(uint4 hv, uint4 lv, int row, int sg, float* f, uint16_t* h, uint16_t* l) {
+  constexpr int kLDF = Chunk<CK>::LDF, kLDH = Chunk<CK>::LDH;
+  const bf16x2 olo = bf16_pair_bits(kBf16OneLo), ohi = bf16_pair_bits(kBf16OneHi);
+  if (f) {
+    float4* dst = reinterpret_cast<float4*>(f + row * kLDF + sg * 8);
+    dst[0] = make_float4(bf_sum_lo(hv.x, lv.x, olo), bf_sum_hi(hv.x, lv.x, ohi),
+                         bf_sum_lo(hv.y, lv.y, olo), bf_sum_hi(hv.y, lv.y, ohi));
+    dst[1] = make_float4(bf_sum_lo(hv.z, lv.z, olo), bf_sum_hi(hv.z, lv.z, ohi),
+                         bf_sum_lo(hv.w, lv.w, olo), bf_sum_hi(hv.w, lv.w, ohi));
+  }
+  if (h) {
+    // cells 8s+4q..8s+4q+3 of the K step (s = sg % 4, q = 0, 1) go to
+    // 16(s & 1) + 8q + 4(s >> 1)
+    const int base = row * kLDH + (sg & ~3) * 8 + 16 * (sg & 1) + 4 * ((sg >> 1) & 1);
+    *reinterpret_cast<uint2*>(h + base) = make_uint2(hv.x, hv.y);
+    *reinterpret_cast<uint2*>(h + base + 8) = make_uint2(hv.z, hv.w);
+    *reinterpret_cast<uint2*>(l + base) = make_uint2(lv.x, lv.y);
+    *reinterpret_cast<uint2*>(l + base + 8) = make_uint2(lv.z, lv.w);
+  }
+}
+
+// Every row below n.
 template <int CK, int PV>
 BSK_DEV void put(const Pref<PV>& p, int n, float* f, uint16_t* h, uint16_t* l) {
-  constexpr int kSEGS = Chunk<CK>::SEGS, kLDF = Chunk<CK>::LDF, kLDH = Chunk<CK>::LDH;
-  const bf16x2 olo = bf16_pair_bits(kBf16OneLo), ohi = bf16_pair_bits(kBf16OneHi);
+  constexpr int kSEGS = Chunk<CK>::SEGS;
 #pragma unroll
   for (int k = 0; k < PV; ++k) {
     const int v = threadIdx.x + k * kNT;
-    if (v < n * kSEGS) {
-      const int row = v / kSEGS, sg = v - row * kSEGS;
-      const uint4 hv = p.h[k], lv = p.l[k];
-      if (f) {
-        float4* dst = reinterpret_cast<float4*>(f + row * kLDF + sg * 8);
-        dst[0] = make_float4(bf_sum_lo(hv.x, lv.x, olo), bf_sum_hi(hv.x, lv.x, ohi),
-                             bf_sum_lo(hv.y, lv.y, olo), bf_sum_hi(hv.y, lv.y, ohi));
-        dst[1] = make_float4(bf_sum_lo(hv.z, lv.z, olo), bf_sum_hi(hv.z, lv.z, ohi),
-                             bf_sum_lo(hv.w, lv.w, olo), bf_sum_hi(hv.w, lv.w, ohi));
-      }
-      if (h) {
-        // cells 8s+4q..8s+4q+3 of the K step (s = sg % 4, q = 0, 1) go to
-        // 16(s & 1) + 8q + 4(s >> 1)
-        const int base = row * kLDH + (sg & ~3) * 8 + 16 * (sg & 1) + 4 * ((sg >> 1) & 1);
-        *reinterpret_cast<uint2*>(h + base) = make_uint2(hv.x, hv.y);
-        *reinterpret_cast<uint2*>(h + base + 8) = make_uint2(hv.z, hv.w);
-        *reinterpret_cast<uint2*>(l + base) = make_uint2(lv.x, lv.y);
-        *reinterpret_cast<uint2*>(l + base + 8) = make_uint2(lv.z, lv.w);
-      }
-    }
+    if (v < n * kSEGS) put_segment<CK>(p.h[k], p.l[k], v / kSEGS, v % kSEGS, f, h, l);
+  }
+}
+
+template <int CK, int PV>
+BSK_DEV void put(const Pref<PV>& p, const RowSet<PV>& q, float* f, uint16_t* h, uint16_t* l) {
+  constexpr int kSEGS = Chunk<CK>::SEGS;
+  const int sg = threadIdx.x % kSEGS;
+#pragma unroll
+  for (int k = 0; k < PV; ++k) {
+    if (q.r[k] < 0) continue;
+    const int row = q.r[k] & 0xffff;
+    if (f && (int)(threadIdx.x + k * kNT) / kSEGS < q.nf)
+      put_segment<CK>(p.h[k], p.l[k], row, sg, f, nullptr, nullptr);
+    if (h && (q.r[k] >> 16 & 1)) put_segment<CK>(p.h[k], p.l[k], row, sg, nullptr, h, l);
   }
 }
 
@@ -183,6 +227,93 @@ __global__ __launch_bounds__(kNT, (pair_occupancy<NI, PV, SETS, D2>())) void k_t
   const int lane = threadIdx.x & 63;
   const int col = lane & 15, grp = lane >> 4;
 
+  // the cell range (lw) and item-list pass of this workgroup
+  int lw = blockIdx.x, pass = 0;
+  if (a.npass > 1) {
+    pass = (blockIdx.x >> 3) % a.npass;
+    lw = (blockIdx.x / (8 * a.npass)) * 8 + (blockIdx.x & 7);
+  }
+  // item descriptors and partial positions of this wave and the LDS rows of
+  // this lane's pair
+  int desc[NI], oij[NI], opos[NI];
+  setup<NI, kLDF>(desc, oij, opos, a.items + pass * a.pass_stride,
+                  a.outpos + pass * a.pass_stride, a.pairs, wave, col, a.lo_row, n0);
+
+  // the rows that the workgroup's items read: marks of pair sides (sets 0 and
+  // 1) and third-side blocks in LDS, from them each thread's rows (at most 128
+  // shells: two per lane of a wave).  Launches of a single pass read nearly
+  // every row they stage, and those of few shells lose more by the set-up than
+  // they save (a batch of 14 pairs on small meshes 1320 -> 1369 us): they
+  // stage every row.
+  constexpr bool kRows = PV >= 2;
+  std::conditional_t<kRows, RowSet<PV>, int> q0, q1, q2;
+  if constexpr (!kRows) {
+    q0 = n0;
+    q1 = n1;
+    q2 = n2;
+  } else if (a.npass == 1) {
+    auto all = [&](RowSet<PV>& q, int n) {
+      q.nf = n;
+#pragma unroll
+      for (int k = 0; k < PV; ++k) {
+        const int i = (int)(threadIdx.x + k * kNT) / Chunk<CK>::SEGS;
+        q.r[k] = i < n ? i | 1 << 16 : -1;
+      }
+    };
+    all(q0, n0);
+    if (SETS == 3) all(q1, n1);
+    if (SETS >= 2) all(q2, n2);
+  } else {
+    int* const mark = reinterpret_cast<int*>(smem);
+    int* const mark1 = mark + n0 + 1;
+    int* const blk = mark1 + n1 + 1;
+    int* const list = blk + 17;
+    for (int e = threadIdx.x; e < n0 + n1 + 19; e += kNT) mark[e] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < NI; ++s)
+      if (!(desc[s] & (1 << 29)) && grp == 0) {
+        mark[(oij[s] & 0xffff) / kLDF] = 1;
+        (SETS == 3 ? mark1 : mark)[((unsigned)oij[s] >> 16) / kLDF] = 1;
+        if (col == 0) blk[(desc[s] >> 16) & 0xff] = 1;
+      }
+    __syncthreads();
+    auto build = [&](RowSet<PV>& q, int n, const int* pair, bool third) {
+      unsigned long long bp[2], bt[2];
+      int t[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int row = lane + 64 * e;
+        const bool p = row < n && pair && pair[row];
+        t[e] = row < n && third && blk[(row + a.koff) >> 4];
+        bp[e] = __ballot(p);
+        bt[e] = __ballot(t[e] && !p);
+      }
+      q.nf = __popcll(bp[0]) + __popcll(bp[1]);
+      const int total = q.nf + __popcll(bt[0]) + __popcll(bt[1]);
+      const unsigned long long below = (1ull << lane) - 1;
+      if (wave == 0)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const int v = (lane + 64 * e) | (t[e] << 16);
+          if (bp[e] >> lane & 1)
+            list[__popcll(bp[e] & below) + (e ? __popcll(bp[0]) : 0)] = v;
+          else if (bt[e] >> lane & 1)
+            list[q.nf + __popcll(bt[e] & below) + (e ? __popcll(bt[0]) : 0)] = v;
+        }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < PV; ++k) {
+        const int i = (int)(threadIdx.x + k * kNT) / Chunk<CK>::SEGS;
+        q.r[k] = i < total ? list[i] : -1;
+      }
+      __syncthreads();
+    };
+    build(q0, n0, mark, SETS == 1);
+    if (SETS == 3) build(q1, n1, mark1, false);
+    if (SETS >= 2) build(q2, n2, nullptr, true);
+  }
+
   // zero rows: FP32 padding rows and the third-side rows outside the staged
   // shells [koff, koff + n2)
   for (int e = threadIdx.x; e < kLDF; e += kNT) {
@@ -199,17 +330,6 @@ __global__ __launch_bounds__(kNT, (pair_occupancy<NI, PV, SETS, D2>())) void k_t
   uint16_t* const hKs = hK + a.koff * kLDH;  // row of staged third-side shell 0
   uint16_t* const lKs = lK + a.koff * kLDH;
 
-  // the cell range (lw) and item-list pass of this workgroup
-  int lw = blockIdx.x, pass = 0;
-  if (a.npass > 1) {
-    pass = (blockIdx.x >> 3) % a.npass;
-    lw = (blockIdx.x / (8 * a.npass)) * 8 + (blockIdx.x & 7);
-  }
-  // item descriptors and partial positions of this wave and the LDS rows of
-  // this lane's pair
-  int desc[NI], oij[NI], opos[NI];
-  setup<NI, kLDF>(desc, oij, opos, a.items + pass * a.pass_stride,
-                  a.outpos + pass * a.pass_stride, a.pairs, wave, col, a.lo_row, n0);
   State<NI> st;
   init(st);
 
@@ -255,21 +375,21 @@ __global__ __launch_bounds__(kNT, (pair_occupancy<NI, PV, SETS, D2>())) void k_t
   } else {
     Pref<PV> p0, p1, p2;
     if (ch0 < ch1) {
-      fetch<CK>(p0, a.hi[0], a.lo[0], a.stride, n0, ch0 * kCK);
-      if (SETS == 3) fetch<CK>(p1, a.hi[1], a.lo[1], a.stride, n1, ch0 * kCK);
-      if (SETS >= 2) fetch<CK>(p2, a.hi[2], a.lo[2], a.stride, n2, ch0 * kCK);
+      fetch<CK>(p0, q0, a.hi[0], a.lo[0], a.stride, ch0 * kCK);
+      if (SETS == 3) fetch<CK>(p1, q1, a.hi[1], a.lo[1], a.stride, ch0 * kCK);
+      if (SETS >= 2) fetch<CK>(p2, q2, a.hi[2], a.lo[2], a.stride, ch0 * kCK);
     }
     for (long long ch = ch0; ch < ch1; ++ch) {
       __syncthreads();  // every wave is done with the previous chunk
-      put<CK>(p0, n0, fA, SETS == 1 ? hKs : nullptr, SETS == 1 ? lKs : nullptr);
-      if (SETS == 3) put<CK>(p1, n1, fB, nullptr, nullptr);
-      if (SETS >= 2) put<CK>(p2, n2, nullptr, hKs, lKs);
+      put<CK>(p0, q0, fA, SETS == 1 ? hKs : nullptr, SETS == 1 ? lKs : nullptr);
+      if (SETS == 3) put<CK>(p1, q1, fB, nullptr, nullptr);
+      if (SETS >= 2) put<CK>(p2, q2, nullptr, hKs, lKs);
       __syncthreads();
       if (ch + 1 < ch1) {  // next chunk's HBM loads overlap this chunk's math
         const long long cb = (ch + 1) * kCK;
-        fetch<CK>(p0, a.hi[0], a.lo[0], a.stride, n0, cb);
-        if (SETS == 3) fetch<CK>(p1, a.hi[1], a.lo[1], a.stride, n1, cb);
-        if (SETS >= 2) fetch<CK>(p2, a.hi[2], a.lo[2], a.stride, n2, cb);
+        fetch<CK>(p0, q0, a.hi[0], a.lo[0], a.stride, cb);
+        if (SETS == 3) fetch<CK>(p1, q1, a.hi[1], a.lo[1], a.stride, cb);
+        if (SETS >= 2) fetch<CK>(p2, q2, a.hi[2], a.lo[2], a.stride, cb);
       }
       ksteps();
     }
