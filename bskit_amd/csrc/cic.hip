@@ -27,7 +27,7 @@
 //     its T^3 nodes into fixed point in LDS: of its own particles and of those
 //     classes of the seven tiles below that reach it (1.2 records per particle
 //     in all), then writes its nodes as float.
-// 256^3 particles on 512^3: 0.55 ms (bin 155 us, place 153, tile 213: the LDS
+// 256^3 particles on 512^3: 0.53 ms (bin 161 us, place 144, tile 219: the LDS
 // atomics; 0.8 GB cross HBM at least).  Tiles that summed only their own
 // particles, wrote the shared face nodes to a boundary record of 400 MB and left
 // them to a pass of its own took 375 + 329 us for the tile step.
