@@ -702,7 +702,8 @@ class GridEngine:
                 cells = (ctypes.c_longlong * L.LEVELS)(*lay.ncell)
             nbytes = L.size_out()
             L.call('bsk_triples_mfma_workspace', plan.handle, nwg, ctypes.byref(nbytes))
-            w = (work or self.work).get('mfma', nbytes.value)
+            # not 'mfma': split-BF16 sums of this engine may be in flight on another stream
+            w = (work or self.work).get('pairs64', nbytes.value)
             L.call('bsk_triples_f64', plan.handle, L.ptr(sa.data), L.ptr(sb.data), L.ptr(sc.data),
                    sa.stride, sa.sum_cells, off, cells, None, nwg, float(scale), L.ptr(out),
                    L.ptr(w), s)
@@ -889,7 +890,7 @@ class GridEngine:
             part = torch.empty(4 * T, dtype=torch.float64, device=self.device)
             L.call('bsk_triples_f64', plan.handle, None, L.ptr(buf), None, n, n, None, None,
                    L.ptr(buf[2 * nb]), nwg, 1.0, L.ptr(part),
-                   L.ptr(self.work.get('mfma', size.value)), s)
+                   L.ptr(self.work.get('gi_t', size.value)), s)
             total = part if total is None else total + part
         return total
 
