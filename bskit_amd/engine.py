@@ -839,11 +839,14 @@ class GridEngine:
         if max_bytes is None:
             free, _ = torch.cuda.mem_get_info(self.device)
             max_bytes = int(free * 0.5)
-        if self.pairs64_supported(2 * self.nb, 1):
-            total = self._gridinfo_wedge(tri, max_bytes, stream)
-        else:
-            total = self._gridinfo_tiled(tri, max_bytes, stream)
-        sums = (total / float(self.ncell)).view(T, 4).cpu().numpy()
+        # kernels, buffers, additions and the copy to the host all on one
+        # stream: the copy waits for them, and the buffers return to its pool
+        with torch.cuda.stream(stream):
+            if self.pairs64_supported(2 * self.nb, 1):
+                total = self._gridinfo_wedge(tri, max_bytes)
+            else:
+                total = self._gridinfo_tiled(tri, max_bytes)
+            sums = (total / float(self.ncell)).view(T, 4).cpu().numpy()
         ntri = np.rint(sums[:, 0])
         kbar = np.full((T, 3), np.nan)
         nz = ntri != 0
@@ -855,7 +858,7 @@ class GridEngine:
         L.call('bsk_gridinfo_layout', self._plan, x0, x1, ctypes.byref(n), ctypes.byref(nbytes))
         return n.value, nbytes.value
 
-    def _gridinfo_wedge(self, tri, max_bytes, stream):
+    def _gridinfo_wedge(self, tri, max_bytes):
         """The four sums of each triangle over the S^3 mesh, from the wedge."""
         T, nb = len(tri), self.nb
         key = (np.ascontiguousarray(tri).tobytes(), 'gridinfo')
@@ -874,7 +877,7 @@ class GridEngine:
                     break
                 x1 = x0 + max(1, (x1 - x0) // 2)
             cuts.append(x1)
-        s = stream_handle(stream)
+        s = stream_handle()
         total = None
         for x0, x1 in zip(cuts[:-1], cuts[1:]):
             n, nbytes = self._gridinfo_slab(x0, x1)
@@ -894,7 +897,7 @@ class GridEngine:
             total = part if total is None else total + part
         return total
 
-    def _gridinfo_tiled(self, tri, max_bytes, stream):
+    def _gridinfo_tiled(self, tri, max_bytes, stream=None):
         """The same sums x slab by x slab of the whole mesh with the tiled FP64
         kernel, for more shells than the pair kernel holds."""
         T = len(tri)

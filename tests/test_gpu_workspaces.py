@@ -78,3 +78,27 @@ def test_side_by_side():
         assert np.array_equal(o.cpu().numpy(), a)
     assert np.array_equal(b1.cpu().numpy(), b)
     assert np.array_equal(n1, n0) and np.array_equal(k1, k0, equal_nan=True)
+
+
+@pytest.mark.parametrize('nb', [16, 140])  # wedge; more shells than it takes
+def test_grid_info_stream(nb):
+    """grid_info on a stream that still has work queued: its kernels, sums and
+    copy to the host wait for it and for each other."""
+    if nb == 16:
+        eng, _, tri = setup(128, nb)
+    else:
+        kf = 2 * np.pi / 1000.0
+        low = kf * (1 + 0.1 * np.arange(nb))
+        eng = GridEngine(48, 1000.0, low, low + 0.1 * kf)
+        tri = np.array([[0, 0, 0], [139, 130, 20], [60, 60, 60]], np.int32)
+    want = [eng.grid_info(tri, max_bytes=b) for b in (1 << 22, None)]  # several slabs; one
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        x = torch.ones((4096, 4096), device='cuda')
+        for _ in range(20):
+            x = x @ x
+            x /= x.max()
+    for (n0, k0), b in zip(want, (1 << 22, None)):
+        n1, k1 = eng.grid_info(tri, max_bytes=b, stream=side)
+        assert np.array_equal(n1, n0) and np.array_equal(k1, k0, equal_nan=True)
