@@ -68,11 +68,12 @@ BSK_DEV void particle(const float* __restrict__ pos, long long p, int N, float t
 // fixed-point weight of corner c (bit 2: x+1, bit 1: y+1, bit 0: z+1): w 2^32
 // rounded to nearest even, as the integer the FP64 sum with 1.5 2^52 holds in
 // its low bits (0 <= w <= 1; a conversion to 64-bit integers is many more
-// instructions)
+// instructions).  A particle at a non-finite position has NaN fractions and
+// weighs nothing: the maximum with 0 takes the number, not the NaN.
 BSK_DEV unsigned long long corner_weight(const float (&f)[3], int c) {
   const float w = ((c & 4) ? f[0] : 1.f - f[0]) * ((c & 2) ? f[1] : 1.f - f[1]) *
                   ((c & 1) ? f[2] : 1.f - f[2]);
-  const double m = __builtin_fma((double)w, kFix, 0x1.8p52);
+  const double m = __builtin_fma((double)fmaxf(w, 0.f), kFix, 0x1.8p52);
   return (unsigned long long)(__double_as_longlong(m) - 0x4338000000000000ll);
 }
 

@@ -402,7 +402,8 @@ int bsk_triples_zfused(bsk_plan* plan, const bsk_pairs* pairs, const void* shell
  * Mesh node i sits at i*box/nmesh.  With to_contrast the result is
  * delta = rho/rho_mean - 1.  Every corner weight is rounded once to 32.32
  * fixed point and summed as integers, so the mesh is the same bits whatever
- * order the particles are processed in (deterministic).  Replaces nbodykit's
+ * order the particles are processed in (deterministic); a particle at a
+ * non-finite position adds nothing.  Replaces nbodykit's
  * CatalogSource.to_mesh(window='cic') painting as called by
  * scripts/measure/measure_bs_fast.py:209-217 (the compensation is
  * bsk_plan_set_compensation).  work: bsk_cic_workspace() bytes; at most
