@@ -958,8 +958,12 @@ class GridEngine:
         return fmt == L.FMT_BF16X2 and self.levels and self.layout is not None
 
     def levels64(self):
-        """Whether FP64 pair sums run over the level layout of this mesh."""
-        return self.levels and self.layout is not None and self.S >= F64_LEVELS_MESH
+        """Whether FP64 pair sums run over the level layout of this mesh: from
+        F64_LEVELS_MESH up, while a row of it stays below the 4 GiB that the z
+        pass addresses in that layout (a 1024^3 mesh's does not; in C order a
+        row may be longer)."""
+        return (self.levels and self.layout is not None and self.S >= F64_LEVELS_MESH and
+                self.layout.stride * 8 < 1 << 32)
 
     def shell_bytes(self, fmt, nb=None):
         """Device bytes of a default shell set (alloc_shells) of nb shells."""
