@@ -33,6 +33,7 @@
 // branch on the tile's pair mask).
 #include <algorithm>
 #include <array>
+#include <climits>
 #include <new>
 #include <vector>
 
@@ -457,6 +458,14 @@ void make_tables(BlockTables& t, const int set[3], const std::vector<Tri>& tri) 
 // Rows of partial sums held at a time: longer lists run in several launches.
 constexpr int kRowBatch = 16384;
 
+// Groups of one launch: either kernel runs 4096 threads per group and chunk,
+// and a launch dimension holds less than 2^32 threads (lists whose groups hold
+// few triangles pass that before kRowBatch rows: 255 groups at 4096 chunks).
+constexpr long long kGroupThreads = 64 * kWaves * kLaneGroups;
+int group_batch(int nchunk) {
+  return (int)std::min<long long>(INT_MAX, 0xffffffffLL / (8LL * ((nchunk + 7LL) / 8) * kGroupThreads));
+}
+
 template <int BS, bool STAGED>
 int launch_blocked(const BlockTables& t, BlockedArgs a, double scale, double* out, hipStream_t s) {
   constexpr int ST = 2;
@@ -469,14 +478,14 @@ int launch_blocked(const BlockTables& t, BlockedArgs a, double scale, double* ou
   for (int g0 = 0; g0 < t.ngroup;) {
     const int r0 = g0 ? t.row_end[g0 - 1] : 0;
     int g1 = g0 + 1;
-    while (g1 < t.ngroup && t.row_end[g1] - r0 <= kRowBatch) ++g1;
+    while (g1 < t.ngroup && g1 - g0 < group_batch(a.nchunk) && t.row_end[g1] - r0 <= kRowBatch) ++g1;
     const int r1 = t.row_end[g1 - 1];
     const int e0 = r0 ? t.entry_end[r0 - 1] : 0, e1 = t.entry_end[r1 - 1];
     a.ngroup = g1 - g0;
     a.tabs = t.d_tabs + (size_t)g0 * Tab<BS>::ints;
     a.rows = t.d_rows + (size_t)g0 * kWaves * BS * BS * BS;
     a.row0 = r0;
-    const unsigned per_xcd = (unsigned)((a.nchunk + 7) / 8);
+    const unsigned per_xcd = ((unsigned)a.nchunk + 7) / 8;
     if constexpr (STAGED)
       hipLaunchKernelGGL((k_triple_blocked<BS, ST>), dim3(8u * per_xcd * a.ngroup * kLaneGroups),
                          dim3(64 * kWaves), lds, s, a);
@@ -501,9 +510,10 @@ int launch_blocked(const BlockTables& t, BlockedArgs a, double scale, double* ou
 //    direct reads its tiles' shells from the caches at about 15 TB/s.  512^3,
 //    3624 triangles 42400 / 4660 / 1780; 256^3, 564 triangles (62 chunks) 3200 /
 //    400 / 245; <ABC>, 407 triangles over 64^3 cells 63 / 43 / 120.
+// A launch of direct or blocked must hold one group at least (group_batch).
 enum Way { kPlain, kDirect, kStaged };
 Way pick(const bsk_blocked* q, long long ncell, int nchunk) {
-  if (q->nrow < 2 * q->t2.ntile) return kPlain;
+  if (q->nrow < 2 * q->t2.ntile || !group_batch(nchunk)) return kPlain;
   const long long groups = (long long)q->t4.ngroup * nchunk * kLaneGroups;
   const double blocked = 125.0 * (double)((groups + 255) / 256) * ((double)ncell / nchunk / 65536.0);
   const double direct = (double)q->t2.ntile * (double)ncell * (6 * sizeof(float)) / 15e6;
