@@ -250,15 +250,16 @@ __device__ constexpr CicRun kRun[kRuns] = {
     {0, 0, 7}, {4, 4, 7}, {2, 2, 3}, {2, 6, 7}, {1, 1, 1}, {1, 3, 3}, {1, 5, 5},
     {1, 7, 7}, {6, 6, 7}, {5, 5, 5}, {5, 7, 7}, {3, 3, 3}, {3, 7, 7}, {7, 7, 7}};
 
+// grid (tiles of an x layer, x layers): one dimension would pass 2^32 threads
+// from N = 3264 up
 constexpr int kTW = 512;  // threads per tile (284 us with 256)
 __global__ __launch_bounds__(kTW) void k_cic_tile(const CicRec* __restrict__ rec,
                                                   const uint32_t* __restrict__ off, int N,
                                                   double scale, float shift,
                                                   float* __restrict__ grid) {
   __shared__ unsigned long long acc[kT * kT * kT];
-  const int tile = blockIdx.x;
   const int nt = N / kT;
-  const int tx = tile / (nt * nt), ty = (tile / nt) % nt, tz = tile % nt;
+  const int tx = blockIdx.y, ty = blockIdx.x / nt, tz = blockIdx.x % nt;
   for (int i = threadIdx.x; i < kT * kT * kT; i += kTW) acc[i] = 0ull;
   // the runs one after the other: entry e of them is record start[r] + e,
   // r the last run with begin[r] <= e
@@ -438,8 +439,9 @@ extern "C" int bsk_cic_paint(int nmesh, double box_size, long long npart, const 
                        off, slot, rec);
     BSK_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(k_cic_tile, dim3((unsigned)(w.nbin / kClass)), dim3(kTW), 0, s, rec, off,
-                     nmesh, scale, shift, grid);
+  const unsigned nt = nmesh / kT;
+  hipLaunchKernelGGL(k_cic_tile, dim3(nt * nt, nt), dim3(kTW), 0, s, rec, off, nmesh, scale, shift,
+                     grid);
   BSK_LAUNCH_CHECK();
   return BSK_OK;
 }
