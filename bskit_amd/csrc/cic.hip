@@ -31,8 +31,9 @@
 // atomics; 0.8 GB cross HBM at least).  Tiles that summed only their own
 // particles, wrote the shared face nodes to a boundary record of 400 MB and left
 // them to a pass of its own took 375 + 329 us for the tile step.
-// Other N: fixed-point 64-bit atomics into an N^3 integer workspace, then a
-// conversion pass (same integers, so the same bits as the tiled path).
+// Other N (and 2^29 or more particles on one tile): fixed-point 64-bit atomics
+// into an N^3 integer workspace, then a conversion pass (same integers, so the
+// same bits as the tiled path).
 #include <algorithm>
 
 #include "common.h"
@@ -334,7 +335,12 @@ __global__ __launch_bounds__(256) void k_cic_convert(const unsigned long long* _
     grid[i] = node_value(acc[i], scale, shift);
 }
 
-bool tiled(int nmesh) { return nmesh % kT == 0; }
+// A mesh of one tile reads a record of class 7 eight times over (its own
+// neighbour on every side), which 32-bit record counts hold below 2^29
+// particles; with more tiles a side no tile reads a record twice.
+bool tiled(int nmesh, long long npart) {
+  return nmesh % kT == 0 && (nmesh > kT || npart < (1ll << 29));
+}
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
@@ -369,7 +375,7 @@ extern "C" int bsk_cic_workspace(int nmesh, long long npart, size_t* bytes) {
     bsk_set_error("bsk_cic_workspace: at most 2^32 - 1 particles");
     return BSK_EINVAL;
   }
-  if (tiled(nmesh))
+  if (tiled(nmesh, npart))
     *bytes = tiled_ws(nmesh, npart).total;
   else
     *bytes = (size_t)nmesh * nmesh * nmesh * 8;
@@ -399,7 +405,7 @@ extern "C" int bsk_cic_paint(int nmesh, double box_size, long long npart, const 
   const float shift = to_contrast ? 1.f : 0.f;
   const unsigned pblocks = (unsigned)((npart + 255) / 256);
   char* wb = static_cast<char*>(work);
-  if (!tiled(nmesh)) {
+  if (!tiled(nmesh, npart)) {
     auto* acc = reinterpret_cast<unsigned long long*>(wb);
     hipLaunchKernelGGL(k_fill_u64, dim3(4096), dim3(256), 0, s, acc, ncell);
     BSK_LAUNCH_CHECK();
