@@ -841,6 +841,7 @@ struct bsk_pairs {
   int seg_ni[kParts] = {1, 1, 1, 1};  // items per wave of the segment's launches
   int seg_rep[kParts] = {1, 1, 1, 1};  // replicas of its wave lists (each runs 1/rep of the K steps)
   int item_total = 0;  // distinct items: partial positions per workgroup
+  std::vector<int> pass_item;  // FP64: items before each pass (all segments'), and in all
   std::vector<int> slot;  // [ntri][kParts]: each triangle's slot per segment, -1 for none
   std::vector<int> h_items, h_outpos, h_pairs;
   int* d_items = nullptr;   // per launch [waves * ni of its segment]; owns the tables' block
@@ -1265,6 +1266,20 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
   }
   int npass = 0;
   for (const auto& g : sp) npass += g.npass;
+  // FP64 partials are kept and reduced a few passes at a time: positions in
+  // the order of the passes
+  std::vector<int> pass_item;
+  if (f64) {
+    int pos = 0;
+    for (const auto& g : sp)
+      for (size_t b = 0; b < g.bins.size(); ++b) {
+        if (b % W == 0) pass_item.push_back(pos);
+        for (int u : g.bins[b])
+          for (int kb = 0; kb < nkb; ++kb)
+            if (g.unit_mask[u] >> kb & 1u) item_of[(size_t)g.unit_tile[u] * nkb + kb] = pos++;
+      }
+    pass_item.push_back(pos);
+  }
   // launch lists: descriptors tile | kb << 16 | padding << 29 | (first item
   // of a unit: new pair products) << 31, kb counted from the segment's first
   // staged block; partial positions (-1: padding); each launch holds waves x
@@ -1356,6 +1371,7 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
     q->seg_rep[g] = sp[g].rep;
   }
   q->item_total = std::max(nitem, 1);
+  q->pass_item.swap(pass_item);
   q->h_items.swap(items);
   q->h_outpos.swap(outpos);
   q->h_pairs.swap(prs);
@@ -1462,13 +1478,47 @@ int bsk_pairs_tables(const bsk_pairs* q, int* items, int* outpos, int* pairs) {
   return BSK_OK;
 }
 
+}  // extern "C"
+
+namespace {
+// FP64 partials (2 KB per item and workgroup) held at a time: the passes of a
+// list run in batches of at most this (one pass at least), each reduced before
+// the next.  All of a list's at once took 1.0 GB for 80 bins of 256^3 (49533
+// triangles) and 3.9 GB for 130 bins of 400^3, and the passes of one launch
+// gained nothing by it: 13.18 and 177.9 ms, in batches of 1 GB 13.19 and 180.3,
+// of 256 MB 13.10 and 177.4, of 128 MB 12.91 and 176.9.
+constexpr size_t kDPairPartials = (size_t)128 << 20;
+
+// End of the batch of passes that begins with pass p0.
+int dpair_batch(const bsk_pairs* q, int nwg, int p0) {
+  const long long most = (long long)(kDPairPartials / (2048 * (size_t)nwg));
+  const int np = (int)q->pass_item.size() - 1;
+  int p1 = p0 + 1;
+  while (p1 < np && q->pass_item[p1 + 1] - q->pass_item[p0] <= most) ++p1;
+  return p1;
+}
+
+// Partial positions of the largest batch.
+int dpair_batch_items(const bsk_pairs* q, int nwg) {
+  int most = 1;
+  for (int p = 0; p + 1 < (int)q->pass_item.size();) {
+    const int e = dpair_batch(q, nwg, p);
+    most = std::max(most, q->pass_item[e] - q->pass_item[p]);
+    p = e;
+  }
+  return most;
+}
+}  // namespace
+
+extern "C" {
+
 int bsk_triples_mfma_workspace(const bsk_pairs* q, int nwg, size_t* bytes) {
   if (!q || nwg <= 0 || !bytes) {
     bsk_set_error("bsk_triples_mfma_workspace: invalid argument");
     return BSK_EINVAL;
   }
   if (q->f64) {
-    *bytes = sizeof(double) * 256 * (size_t)q->item_total * nwg +
+    *bytes = sizeof(double) * 256 * (size_t)dpair_batch_items(q, nwg) * nwg +
              bsk_reduce_dpairs_bytes(q->item_total);
     return BSK_OK;
   }
@@ -1897,34 +1947,46 @@ int bsk_triples_f64(const bsk_pairs* q, const double* f_i, const double* f_j, co
   a.nwg = nwg;
   a.pairs = q->d_pairs;
   a.partial = reinterpret_cast<double*>(work);
-  a.item_total = q->item_total;
+  double* sums = a.partial + (size_t)256 * dpair_batch_items(q, nwg) * nwg;
   hipStream_t s = as_stream(stream);
-  size_t e0 = 0;  // first list entry of the launch
-  for (int g = 0; g < q->nseg; ++g) {  // as triples_mfma's
-    const int fp = __builtin_ctz(q->seg_parts[g]), lp = 31 - __builtin_clz(q->seg_parts[g]);
-    const int w0 = q->seg_win[g][0], wn = q->seg_win[g][1];
-    const long long base = pbeg[fp] + (long long)w0 * shell_stride;
-    for (int r = 0; r < 3; ++r) a.f[r] = f[r] + base;
-    a.weight = weight ? weight + pbeg[fp] : nullptr;
-    a.nsh = wn;
-    a.lo_row = w0;
-    a.koff = w0 % 16;
-    a.nkb = (a.koff + wn + 15) / 16;
-    a.ncell = pend[lp] - pbeg[fp];
-    const int ni = q->seg_ni[g], np = q->seg_pass[g];
-    const bool fold = np > 1 && nwg % 8 == 0;
-    a.npass = fold ? np : 1;
-    a.pass_stride = kPairWaves * ni;
-    for (int k = 0; k < np; k += a.npass) {
+  int g = 0, k = 0;  // segment, and the pass p of the list within it
+  size_t e0 = 0;     // first list entry of the segment
+  const int np = (int)q->pass_item.size() - 1;
+  for (int p0 = 0; p0 < np;) {  // batches of passes
+    const int p1 = dpair_batch(q, nwg, p0);
+    a.item0 = q->pass_item[p0];
+    a.item_total = q->pass_item[p1] - a.item0;
+    for (int p = p0; p < p1;) {  // launches, as triples_mfma's
+      const int fp = __builtin_ctz(q->seg_parts[g]), lp = 31 - __builtin_clz(q->seg_parts[g]);
+      const int w0 = q->seg_win[g][0], wn = q->seg_win[g][1];
+      const long long base = pbeg[fp] + (long long)w0 * shell_stride;
+      for (int r = 0; r < 3; ++r) a.f[r] = f[r] + base;
+      a.weight = weight ? weight + pbeg[fp] : nullptr;
+      a.nsh = wn;
+      a.lo_row = w0;
+      a.koff = w0 % 16;
+      a.nkb = (a.koff + wn + 15) / 16;
+      a.ncell = pend[lp] - pbeg[fp];
+      const int ni = q->seg_ni[g], left = std::min(p1 - p, q->seg_pass[g] - k);
+      a.npass = nwg % 8 == 0 ? left : 1;
+      a.pass_stride = kPairWaves * ni;
       a.items = q->d_items + e0 + (size_t)k * kPairWaves * ni;
       a.outpos = q->d_outpos + e0 + (size_t)k * kPairWaves * ni;
       if (int rc = bsk_triple_dpairs_launch(a, q->sets, ni, s)) return rc;
+      p += a.npass;
+      k += a.npass;
+      if (k == q->seg_pass[g]) {
+        e0 += (size_t)k * kPairWaves * ni;
+        ++g;
+        k = 0;
+      }
     }
-    e0 += (size_t)np * kPairWaves * ni;
+    if (int rc = bsk_reduce_dslots_launch(a.partial, nwg, a.item_total, sums + 256 * (size_t)a.item0,
+                                          q->item_total, s))
+      return rc;
+    p0 = p1;
   }
-  double* sums = a.partial + (size_t)256 * q->item_total * nwg;
-  return bsk_reduce_dpairs_launch(a.partial, nwg, q->item_total, q->ntri, q->d_slot, scale, out_dev,
-                                  sums, s);
+  return bsk_reduce_tri_launch(sums, 256 * q->item_total, q->ntri, q->d_slot, scale, out_dev, s);
 }
 
 }  // extern "C"

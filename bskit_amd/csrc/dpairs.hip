@@ -150,7 +150,7 @@ BSK_DEV void run_items(const DPairArgs& a, double* smem, const int* items, const
   double* const out = a.partial + (long long)lw * a.item_total * 256;
 #pragma unroll
   for (int s = 0; s < CNT; ++s) {
-    const int pos = __builtin_amdgcn_readfirstlane(outpos[s]);
+    const int pos = __builtin_amdgcn_readfirstlane(outpos[s]) - a.item0;
 #pragma unroll
     for (int r = 0; r < 4; ++r) out[(long long)pos * 256 + (4 * r + grp) * 16 + col] = acc[s][r];
   }
@@ -227,9 +227,11 @@ int launch_pv(const DPairArgs& a, int ni, int pv, size_t lds, hipStream_t s) {
   return BSK_EUNSUPPORTED;
 }
 
-// FP64 partials summed over the workgroups of each of kRedSplit ranges.
+// FP64 partials summed over the workgroups of each of kRedSplit ranges (rows of
+// sum_slots in sums).
 __global__ __launch_bounds__(256) void k_reduce_dslots(const double* __restrict__ partial, int nwg,
-                                                       int nslot, double* __restrict__ sums) {
+                                                       int nslot, double* __restrict__ sums,
+                                                       int sum_slots) {
   const int e = blockIdx.x * 256 + threadIdx.x, c = blockIdx.y;
   if (e >= nslot) return;
   const int w0 = (int)((long long)nwg * c / kRedSplit), w1 = (int)((long long)nwg * (c + 1) / kRedSplit);
@@ -239,7 +241,7 @@ __global__ __launch_bounds__(256) void k_reduce_dslots(const double* __restrict_
 #pragma unroll
     for (int k = 0; k < 4; ++k) s[k] += partial[(long long)(w + k) * nslot + e];
   for (; w < w1; ++w) s[0] += partial[(long long)w * nslot + e];
-  sums[(long long)c * nslot + e] = (s[0] + s[1]) + (s[2] + s[3]);
+  sums[(long long)c * sum_slots + e] = (s[0] + s[1]) + (s[2] + s[3]);
 }
 
 }  // namespace
@@ -281,13 +283,11 @@ size_t bsk_reduce_dpairs_bytes(int items_per_wg) {
   return sizeof(double) * kRedSplit * 256 * (size_t)items_per_wg;
 }
 
-int bsk_reduce_dpairs_launch(const double* partial, int nwg, int items_per_wg, int ntri,
-                             const int* slot, double scale, double* out, double* sums,
-                             hipStream_t s) {
-  if (ntri <= 0) return BSK_OK;
-  const int nslot = items_per_wg * 256;
-  hipLaunchKernelGGL(k_reduce_dslots, dim3((nslot + 255) / 256, kRedSplit), dim3(256), 0, s, partial,
-                     nwg, nslot, sums);
+int bsk_reduce_dslots_launch(const double* partial, int nwg, int items_per_wg, double* sums,
+                             int sum_items, hipStream_t s) {
+  if (items_per_wg <= 0) return BSK_OK;
+  hipLaunchKernelGGL(k_reduce_dslots, dim3(items_per_wg, kRedSplit), dim3(256), 0, s, partial, nwg,
+                     items_per_wg * 256, sums, sum_items * 256);
   BSK_LAUNCH_CHECK();
-  return bsk_reduce_tri_launch(sums, nslot, ntri, slot, scale, out, s);
+  return BSK_OK;
 }

@@ -127,7 +127,7 @@ struct DPairArgs {
   const int* outpos;
   const int* pairs;
   double* partial;        // [nwg][item_total][256]
-  int item_total;
+  int item_total, item0;  // positions kept at a time, and the first of them
   int npass, pass_stride;
   const double* weight;   // per cell, or null (one shell set only)
 };
@@ -135,9 +135,10 @@ int bsk_dpair_items_round(int ni);
 bool bsk_dpair_fits(int sets, int nshell);  // registers and LDS hold a launch's shells
 int bsk_triple_dpairs_launch(const DPairArgs& a, int sets, int ni, hipStream_t s);
 size_t bsk_reduce_dpairs_bytes(int items_per_wg);
-int bsk_reduce_dpairs_launch(const double* partial, int nwg, int items_per_wg, int ntri,
-                             const int* slot, double scale, double* out, double* sums,
-                             hipStream_t s);
+// First step of their reduction: the partials of items_per_wg items to their
+// place in the sums of sum_items items (bsk_reduce_tri_launch follows).
+int bsk_reduce_dslots_launch(const double* partial, int nwg, int items_per_wg, double* sums,
+                             int sum_items, hipStream_t s);
 // Second step of both reductions: per triangle the kRedSplit range sums of
 // its slots.
 constexpr int kRedSplit = 16;
