@@ -965,12 +965,24 @@ class GridEngine:
         return (self.levels and self.layout is not None and self.S >= F64_LEVELS_MESH and
                 self.layout.stride * 8 < 1 << 32)
 
-    def shell_bytes(self, fmt, nb=None):
-        """Device bytes of a default shell set (alloc_shells) of nb shells."""
+    def shell_bytes(self, fmt, nb=None, levels=None):
+        """Device bytes of the shell set alloc_shells(fmt, nb, levels) makes."""
         nb = self.nb if nb is None else nb
         per = 8 if fmt == L.FMT_F64 else 4
-        stride = self.layout.stride if self.uses_levels(fmt) else self.ncell
+        if levels is None:
+            levels = self.uses_levels(fmt)
+        stride = self.layout.stride if levels and self.layout is not None else self.ncell
         return nb * stride * per
+
+    def pairs64_bytes(self, tri, nfield):
+        """Device bytes of scratch of the FP64 pair sums of a list over this
+        mesh's default shells."""
+        levels = self.levels64()
+        plan = self.pair_plan(tri, self.nb, _MODE[nfield], levels=levels, f64=True)
+        cells = self.layout.ncell[0] if levels else self.ncell
+        n = L.size_out()
+        L.call('bsk_triples_mfma_workspace', plan.handle, self.pairs64_nwg(cells), ctypes.byref(n))
+        return n.value
 
 
 def cic_paint(positions, nmesh, box_size, to_contrast=True, out=None, stream=None, work=None):

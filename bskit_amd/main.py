@@ -345,7 +345,12 @@ class FFTBispectrum:
         nf = len(self._fields)
         fmt = self._shell_format(kLU, tri)
         free, _ = torch.cuda.mem_get_info(eng.device)
-        if nf <= 2 and nf * eng.shell_bytes(fmt) > self.slab_threshold * free:
+        limit = self.slab_threshold * free
+        pairs64 = fmt == L.FMT_F64 and eng.pairs64_supported(eng.nb, nf)
+        need = nf * eng.shell_bytes(fmt, levels=eng.levels64() if pairs64 else None)
+        if pairs64 and nf <= 2 and limit / 2 < need <= limit:
+            need += eng.pairs64_bytes(tri, nf)  # looked up where it can decide
+        if nf <= 2 and need > limit:
             # the shell sets do not fit in HBM: make and sum them x slab by x
             # slab (each field's spectrum kept, shells never whole)
             meshes = self._meshes()
