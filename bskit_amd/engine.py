@@ -867,23 +867,24 @@ class GridEngine:
             with torch.cuda.device(self.device):
                 plan = self._tri_cache[key] = PairPlan(tri, nb, L.MODE_AUTO, gridinfo=True)
         # x slabs whose shells, weights and intermediates fit max_bytes (one
-        # plane at least)
-        cuts, end = [0], self.S // 2 + 1
-        while cuts[-1] < end:
-            x0, x1 = cuts[-1], end
-            while x1 > x0 + 1:
+        # plane at least), all in the same buffer
+        slabs, x0, end = [], 0, self.S // 2 + 1
+        while x0 < end:
+            x1 = end
+            while True:
                 n, nbytes = self._gridinfo_slab(x0, x1)
-                if nbytes + (2 * nb + 1) * 8 * n <= max_bytes:
+                nbytes += (2 * nb + 1) * 8 * n
+                if x1 == x0 + 1 or nbytes <= max_bytes:
                     break
                 x1 = x0 + max(1, (x1 - x0) // 2)
-            cuts.append(x1)
+            slabs.append((x0, x1, n, nbytes))
+            x0 = x1
         s = stream_handle()
+        buf = torch.empty(max(v[3] for v in slabs) // 8, dtype=torch.float64, device=self.device)
         total = None
-        for x0, x1 in zip(cuts[:-1], cuts[1:]):
-            n, nbytes = self._gridinfo_slab(x0, x1)
-            wk = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
-            buf = torch.empty((2 * nb + 1, n), dtype=torch.float64, device=self.device)
-            L.call('bsk_gridinfo_shells', self._plan, x0, x1, L.ptr(buf), n, L.ptr(buf[2 * nb]),
+        for x0, x1, n, _ in slabs:  # shells, weights and intermediates
+            weight, wk = buf[2 * nb * n:], buf[(2 * nb + 1) * n:]
+            L.call('bsk_gridinfo_shells', self._plan, x0, x1, L.ptr(buf), n, L.ptr(weight),
                    L.ptr(wk), s)
             # at least four 64-cell chunks per workgroup, at most 256 MB of
             # partials (2 KB per item and workgroup)
@@ -892,7 +893,7 @@ class GridEngine:
             L.call('bsk_triples_mfma_workspace', plan.handle, nwg, ctypes.byref(size))
             part = torch.empty(4 * T, dtype=torch.float64, device=self.device)
             L.call('bsk_triples_f64', plan.handle, None, L.ptr(buf), None, n, n, None, None,
-                   L.ptr(buf[2 * nb]), nwg, 1.0, L.ptr(part),
+                   L.ptr(weight), nwg, 1.0, L.ptr(part),
                    L.ptr(self.work.get('gi_t', size.value)), s)
             total = part if total is None else total + part
         return total
