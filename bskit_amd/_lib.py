@@ -146,8 +146,14 @@ def lib():
 
 
 def built():
-    """Whether the library is there to load (host-only helpers have numpy twins)."""
-    return _lib is not None or os.path.exists(LIB_PATH)
+    """Whether the library is there and loads (host-only helpers have numpy
+    twins for where it does not: no HIP runtime, another version)."""
+    if _lib is None:
+        try:
+            lib()
+        except (OSError, ImportError, AttributeError):
+            return False
+    return True
 
 
 def dbl_ptr(a):
