@@ -21,7 +21,7 @@ KIND_DELTA, KIND_UNIT, KIND_KMAG, KIND_KPOW = 0, 1, 2, 3
 MODE_AUTO, MODE_AAB, MODE_ABC = 0, 1, 2
 STAGE_X, STAGE_YZ, STAGE_Y, STAGE_LEVELS = 1, 2, 4, 8
 LEVELS = 4
-ABI_VERSION = 7
+ABI_VERSION = 8
 
 _c_int, _c_ll, _c_double, _vp = ctypes.c_int, ctypes.c_longlong, ctypes.c_double, ctypes.c_void_p
 _c_size_p = ctypes.POINTER(ctypes.c_size_t)
@@ -134,13 +134,14 @@ def lib():
                 raise ImportError('libbskhip.so is not built (%s); run '
                                   '__graft_entry__.build() or make -C %s' % (LIB_PATH, CSRC))
             h = ctypes.CDLL(LIB_PATH)
+            # before the symbols: another version may lack some
+            if h.bsk_version() != ABI_VERSION:
+                raise ImportError('%s has ABI version %d, this package needs %d; rebuild it'
+                                  % (LIB_PATH, h.bsk_version(), ABI_VERSION))
             for name, args in _SIGS.items():
                 fn = getattr(h, name)
                 fn.argtypes = args
                 fn.restype = _RESTYPE.get(name, _c_int)
-            if h.bsk_version() != ABI_VERSION:
-                raise ImportError('%s has ABI version %d, this package needs %d; rebuild it'
-                                  % (LIB_PATH, h.bsk_version(), ABI_VERSION))
             _lib = h
     return _lib
 

@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define BSK_ABI_VERSION 7
+#define BSK_ABI_VERSION 8
 
 /* status codes */
 #define BSK_OK 0

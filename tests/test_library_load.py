@@ -38,3 +38,11 @@ def test_triangle_list_without_library(other_library, kind):
     assert not _lib.built()
     with pytest.raises((OSError, ImportError, AttributeError)):
         _lib.lib()  # the kernels have no twin
+
+
+def test_other_version_is_named(other_library):
+    """A library that lacks newer symbols: the version is what is reported."""
+    compiled(other_library, 'int bsk_version(void) { return 7; }')
+    assert _lib.ABI_VERSION > 7  # 7 was before bsk_closed_triangles and the FP64 pair sums
+    with pytest.raises(ImportError, match='ABI version 7'):
+        _lib.lib()
