@@ -34,7 +34,7 @@
 #include <algorithm>
 #include <array>
 #include <climits>
-#include <new>
+#include <memory>
 #include <vector>
 
 #include "launch.h"
@@ -546,26 +546,29 @@ int bsk_blocked_create(bsk_blocked** out, int mode, int nshell, int ntri, const 
     bsk_set_error("bsk_blocked_create: at most 65535 shells");
     return BSK_EUNSUPPORTED;
   }
-  std::vector<Tri> v(ntri);
-  for (int t = 0; t < ntri; ++t) {
-    for (int e = 0; e < 3; ++e)
-      if (tri[3 * t + e] < 0 || tri[3 * t + e] >= nshell) {
-        bsk_set_error("bsk_blocked_create: triangle %d has a shell index out of range", t);
-        return BSK_EINVAL;
-      }
-    int i = tri[3 * t], j = tri[3 * t + 1];
-    if (mode != BSK_MODE_ABC && i < j) std::swap(i, j);  // d_i d_j of one field: either order
-    v[t] = {{i, j, tri[3 * t + 2]}, t};
-  }
-  bsk_blocked* q = new bsk_blocked();
-  q->ntri = ntri;
-  q->tri.assign(tri, tri + 3 * (size_t)ntri);
-  const int sets[3][3] = {{0, 0, 0}, {0, 0, 2}, {0, 1, 2}};
-  make_tables<4>(q->t4, sets[mode], v);
-  make_tables<2>(q->t2, sets[mode], v);
-  q->nrow = (int)q->t4.entry_end.size();
-  *out = q;
-  return BSK_OK;
+  return bsk_guarded("bsk_blocked_create", [&]() -> int {
+    std::vector<Tri> v(ntri);
+    for (int t = 0; t < ntri; ++t) {
+      const int* s = tri + 3 * (size_t)t;
+      for (int e = 0; e < 3; ++e)
+        if (s[e] < 0 || s[e] >= nshell) {
+          bsk_set_error("bsk_blocked_create: triangle %d has a shell index out of range", t);
+          return BSK_EINVAL;
+        }
+      int i = s[0], j = s[1];
+      if (mode != BSK_MODE_ABC && i < j) std::swap(i, j);  // d_i d_j of one field: either order
+      v[t] = {{i, j, s[2]}, t};
+    }
+    auto q = std::make_unique<bsk_blocked>();
+    q->ntri = ntri;
+    q->tri.assign(tri, tri + 3 * (size_t)ntri);
+    const int sets[3][3] = {{0, 0, 0}, {0, 0, 2}, {0, 1, 2}};
+    make_tables<4>(q->t4, sets[mode], v);
+    make_tables<2>(q->t2, sets[mode], v);
+    q->nrow = (int)q->t4.entry_end.size();
+    *out = q.release();
+    return BSK_OK;
+  });
 }
 
 int bsk_blocked_upload(bsk_blocked* q) {
@@ -574,10 +577,12 @@ int bsk_blocked_upload(bsk_blocked* q) {
     return BSK_EINVAL;
   }
   if (q->d_tri) return BSK_OK;
-  return bsk_upload_tables({&q->tri, &q->t4.tabs, &q->t4.rows, &q->t4.entry, &q->t2.tabs,
-                            &q->t2.rows, &q->t2.entry},
-                           {&q->d_tri, &q->t4.d_tabs, &q->t4.d_rows, &q->t4.d_entry, &q->t2.d_tabs,
-                            &q->t2.d_rows, &q->t2.d_entry});
+  return bsk_guarded("bsk_blocked_upload", [&] {
+    return bsk_upload_tables({&q->tri, &q->t4.tabs, &q->t4.rows, &q->t4.entry, &q->t2.tabs,
+                              &q->t2.rows, &q->t2.entry},
+                             {&q->d_tri, &q->t4.d_tabs, &q->t4.d_rows, &q->t4.d_entry,
+                              &q->t2.d_tabs, &q->t2.d_rows, &q->t2.d_entry});
+  });
 }
 
 int bsk_blocked_destroy(bsk_blocked* q) {

@@ -11,6 +11,7 @@
 #include <array>
 #include <climits>
 #include <cmath>
+#include <memory>
 #include <mutex>
 #include <queue>
 #include <vector>
@@ -1112,9 +1113,8 @@ std::vector<std::vector<int>> bin_units(const std::vector<unsigned>& mask, int c
   return bins;
 }
 
-int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri,
-                 const int* level, const char* fn, bool f64 = false,
-                 const std::vector<Role>* roles = nullptr) {
+int make_pairs(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri, const int* level,
+               const char* fn, bool f64, const std::vector<Role>* roles) {
   if (!out || nshell < 1 || mode < 0 || mode > 2 || ntri < 0 || (ntri && !tri)) {
     bsk_set_error("%s: invalid argument", fn);
     return BSK_EINVAL;
@@ -1311,7 +1311,7 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
   // pair rows in absolute shell indices, 0xffff for padding rows (the
   // kernel's zero row); the last tile is all padding
   std::vector<int> prs((size_t)(ntile + 1) * 16, 0xffff | (0xffff << 16));
-  bsk_pairs* q = new bsk_pairs();
+  auto q = std::make_unique<bsk_pairs>();
   // triangle slots, one per segment (-1: the triangle's level does not
   // include the segment's parts; the first segment holds every triangle)
   q->slot.assign((size_t)kParts * ntri, -1);
@@ -1375,8 +1375,15 @@ int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri
   q->h_items.swap(items);
   q->h_outpos.swap(outpos);
   q->h_pairs.swap(prs);
-  *out = q;
+  *out = q.release();
   return BSK_OK;
+}
+
+int pairs_create(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri,
+                 const int* level, const char* fn, bool f64 = false,
+                 const std::vector<Role>* roles = nullptr) {
+  return bsk_guarded(
+      fn, [&] { return make_pairs(out, mode, nshell, ntri, tri, level, fn, f64, roles); });
 }
 
 }  // namespace
@@ -1433,8 +1440,10 @@ int bsk_pairs_upload(bsk_pairs* q) {
     return BSK_EINVAL;
   }
   if (q->d_items) return BSK_OK;
-  return bsk_upload_tables({&q->h_items, &q->h_outpos, &q->h_pairs, &q->slot},
-                           {&q->d_items, &q->d_outpos, &q->d_pairs, &q->d_slot});
+  return bsk_guarded("bsk_pairs_upload", [&] {
+    return bsk_upload_tables({&q->h_items, &q->h_outpos, &q->h_pairs, &q->slot},
+                             {&q->d_items, &q->d_outpos, &q->d_pairs, &q->d_slot});
+  });
 }
 
 int bsk_pairs_destroy(bsk_pairs* q) {
@@ -1828,29 +1837,31 @@ int bsk_gridinfo_pairs(bsk_pairs** out, int nb, int ntri, const int* tri) {
       bsk_set_error("%s: triangle %d has a shell index out of range", fn, t / 3);
       return BSK_EINVAL;
     }
-  // pairs for the unit-shell sums, then per triangle each side's |k| shell in
-  // the place of its unit shell: on the third side where it may (the pair
-  // products are shared), else on the pair side
-  const std::vector<Role> base = assign_roles_cover(ntri, tri);
-  std::vector<Role> roles((size_t)4 * ntri);
-  std::vector<int> list((size_t)12 * ntri);
-  for (int t = 0; t < ntri; ++t) {
-    const Role r = base[t];
-    roles[4 * (size_t)t] = r;
-    for (int e = 0; e < 3; ++e) {
-      Role& q = roles[4 * (size_t)t + 1 + e] = r;
-      const int v = tri[3 * t + e];
-      if (r.c == v) q.c += nb;
-      else if (r.a == v) q.a += nb;
-      else q.b += nb;
+  return bsk_guarded(fn, [&] {
+    // pairs for the unit-shell sums, then per triangle each side's |k| shell in
+    // the place of its unit shell: on the third side where it may (the pair
+    // products are shared), else on the pair side
+    const std::vector<Role> base = assign_roles_cover(ntri, tri);
+    std::vector<Role> roles((size_t)4 * ntri);
+    std::vector<int> list((size_t)12 * ntri);
+    for (int t = 0; t < ntri; ++t) {
+      const Role r = base[t];
+      roles[4 * (size_t)t] = r;
+      for (int e = 0; e < 3; ++e) {
+        Role& q = roles[4 * (size_t)t + 1 + e] = r;
+        const int v = tri[3 * t + e];
+        if (r.c == v) q.c += nb;
+        else if (r.a == v) q.a += nb;
+        else q.b += nb;
+      }
+      for (int s = 0; s < 4; ++s) {
+        const Role& q = roles[4 * (size_t)t + s];
+        int* l = &list[12 * (size_t)t + 3 * s];
+        l[0] = q.a, l[1] = q.b, l[2] = q.c;
+      }
     }
-    for (int s = 0; s < 4; ++s) {
-      const Role& q = roles[4 * (size_t)t + s];
-      int* l = &list[12 * (size_t)t + 3 * s];
-      l[0] = q.a, l[1] = q.b, l[2] = q.c;
-    }
-  }
-  return pairs_create(out, BSK_MODE_AUTO, 2 * nb, 4 * ntri, list.data(), nullptr, fn, true, &roles);
+    return pairs_create(out, BSK_MODE_AUTO, 2 * nb, 4 * ntri, list.data(), nullptr, fn, true, &roles);
+  });
 }
 
 static int gridinfo_args(const bsk_plan* p, int x0, int x1, GridInfoArgs& a, size_t* bytes) {

@@ -1,5 +1,7 @@
 // Internal host-side launch API shared by the translation units.
 #pragma once
+#include <exception>
+#include <new>
 #include <vector>
 
 #include "common.h"
@@ -11,6 +13,20 @@
   X(16) X(24) X(32) X(40) X(48) X(64) X(72) X(80) X(96) X(120) X(128) X(144) X(160)       \
   X(192) X(200) X(216) X(240) X(256) X(288) X(320) X(384) X(400) X(432) X(480) X(512)    \
   X(576) X(640) X(768) X(1024)
+
+// Body of a C entry that allocates host memory: an exception becomes a status.
+template <typename F>
+int bsk_guarded(const char* fn, F body) {
+  try {
+    return body();
+  } catch (const std::bad_alloc&) {
+    bsk_set_error("%s: out of host memory", fn);
+    return BSK_ENOMEM;
+  } catch (const std::exception& e) {
+    bsk_set_error("%s: %s", fn, e.what());
+    return BSK_EINVAL;
+  }
+}
 
 // Host integer tables in one device block (one allocation and one copy per
 // plan): the tables' device addresses go to where[k], each 16-byte aligned;
