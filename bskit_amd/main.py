@@ -332,9 +332,7 @@ class FFTBispectrum:
                                dtype=torch.float32 if fmt != L.FMT_F64 else torch.float64)
                 self._shells[skey] = s
             sets.append(s)
-        path = {L.FMT_BF16X2: 'mfma', L.FMT_F32: 'blocked',
-                L.FMT_F64: 'pairs64' if pairs64 else 'plain'}[fmt]
-        return sets, path
+        return sets, eng.sum_path(fmt, tri, nf)
 
     def _unnorm_sums(self, kLU, tri, factor):
         """factor * sum_x d_i d_j d_k / ncell: the reference's L^6/N^3 sum
