@@ -26,7 +26,8 @@
 // ones.  Workgroups of a CU turn the lists by one wave each, so that the items
 // of a thin segment (or the ninth of nine) are on different SIMDs.
 //
-// A triangle's sum does not depend on the list it is summed with: its pair is
+// A triangle's sum does not depend on the list this kernel sums it with (lists
+// of a few triangles are faster with one sweep per triangle): its pair is
 // its two largest shells (28 items at 512^3 / 32 bins; the greedy cover of the
 // split-BF16 plans needs 26), every part of the level layout is a segment of
 // its own, the workgroups' cell ranges follow from the mesh, and one wave adds

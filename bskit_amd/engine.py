@@ -603,7 +603,48 @@ class GridEngine:
             return PATH_MFMA
         if fmt == L.FMT_F32:
             return PATH_PLAIN if ntri <= 12 or ntri * ncell <= 3e7 else PATH_BLOCKED
-        return PATH_PAIRS64 if self.pairs64_supported(self.nb, nfield) else PATH_PLAIN
+        if not self.pairs64_supported(self.nb, nfield) or self._short64(tri, nfield, ncell):
+            return PATH_PLAIN
+        return PATH_PAIRS64
+
+    def _short64(self, tri, nfield, ncell):
+        """Whether one sweep per triangle is faster than the FP64 pair kernel,
+        which runs one wave per 16 pairs x 16 third sides of a workgroup's
+        cells: a short list leaves the others idle.
+
+        Estimated times in a measurement, us: one or two sweeps 82, more 100,
+        and 2e-6 for each triangle and cell (more where three shells pass the
+        caches); the pair kernel 72 and 3 for each 64-cell chunk of its 1024
+        workgroups past four, over the sublattices the list's triangles need,
+        and a third more for each further block of 16 third sides (one wave may
+        have to sum both).  Measured, the sums alone on shells in the caches,
+        sweeps / pair kernel: one triangle over all of 480^3 cells 237 / 4200,
+        of 256^3 65 / 686, of 200^3 68 / 362, over a quarter of 200^3 74 / 127,
+        an eighth 70 / 84, of 160^3 71 / 60; over a quarter of 256^3 four 165 /
+        213, eight 335 / 321; over all of 256^3 20 586 / 1123, of 320^3 1476 /
+        2732.  (On small meshes both are latencies: whole measurements with ten
+        triangles over 64^3 cells 209 / 188.)"""
+        ntri = len(tri)
+        if ntri > 24:
+            return False
+        per = 2e-6 if ncell <= 1 << 24 else (2.4e-6 if ncell <= 1 << 25 else 3e-6)
+        sweeps = (82 if ntri <= 2 else 100) + per * ntri * ncell
+        if sweeps > 72 + 6 * max(0.0, ncell / 65536 - 4):
+            return False
+        tri = np.ascontiguousarray(tri, dtype=np.int32)
+        key = (tri.tobytes(), 'short64', nfield, ncell, self.levels64())
+        short = self._tri_cache.get(key)
+        if short is None:
+            part = 1.0
+            if self.levels64():  # C0 minus E, E, O and C1 minus O hold 3, 1, 1 and 3 eighths
+                have = set(self.triangle_levels(tri).tolist())
+                part = sum(n for n, lv in ((3, {0, 1}), (1, have), (1, {0, 2}), (3, {0}))
+                           if have & lv) / 8
+            third = tri.min(axis=1) if nfield == 1 else tri[:, 2]
+            chunk = 3 * (1 + 0.35 * (len(set((third // 16).tolist())) - 1))
+            short = sweeps <= 72 + chunk * max(0.0, part * ncell / 65536 - 4)
+            self._tri_cache[key] = short
+        return short
 
     def plain_nchunk(self, ncell=None):
         ncell = self.ncell if ncell is None else ncell

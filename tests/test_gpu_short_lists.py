@@ -5,7 +5,7 @@ import pytest
 torch = pytest.importorskip('torch')
 import bskit_amd as bsk  # noqa: E402
 from bskit_amd import _lib as L  # noqa: E402
-from bskit_amd.engine import PATH_BLOCKED, PATH_PLAIN, GridEngine  # noqa: E402
+from bskit_amd.engine import PATH_BLOCKED, PATH_PAIRS64, PATH_PLAIN, GridEngine  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 BOX = 1000.0
@@ -39,3 +39,32 @@ def test_fp32_paths(N, nb, cut, monkeypatch):
     tri = fb._fast_bins()[1][7:27]  # 4e7 cells of a 160^3 mesh in two slabs, 3e6 of 64^3
     eng.bispectrum_slabs([dk], tri, path='plain', xslab=eng.S // 2)
     assert paths == 2 * [PATH_PLAIN if N == 64 else PATH_BLOCKED]
+
+
+def test_fp64_paths(monkeypatch):
+    """Short lists by one sweep per triangle, whichever layout the shells have;
+    the sums are the pair kernel's to rounding."""
+    for N, nb, width, cases in ((64, 8, 2, ((1, 0, False), (49, 0, False))),
+                                (256, 16, 3, ((1, 0, False), (4, 0, False), (1, -1, True),
+                                              (18, -18, True), (19, -19, False), (100, 0, False)))):
+        fb = measurement(N, nb, width, torch.float64)
+        eng = fb._engine(fb.bin_edges)
+        n = len(fb.k_edges)
+        assert eng.levels64() == (N == 256)
+        s = fb._shellsets(eng, *fb._fast_bins())[0][0]
+        tri = fb._fast_bins()[1]
+        scale = BOX ** 6 / eng.ncell
+        whole = eng.triples([s], tri, path=PATH_PAIRS64, scale=scale).cpu().numpy()
+        c = eng.shells(eng.forward(fb._fields[0]), fmt=L.FMT_F64, dtype=torch.float64)
+        c.data.abs_()
+        top = eng.triples([c], tri, path=PATH_PLAIN, scale=scale).cpu().numpy()
+        with monkeypatch.context() as m:
+            paths = []
+            triples = eng.triples
+            m.setattr(eng, 'triples', lambda *a, **k: paths.append(k['path']) or triples(*a, **k))
+            for T, at, short in cases:
+                paths.clear()
+                i = at % n
+                got = fb.measure_bispectrum_faster(imin=i, imax=i + T)['B']
+                assert paths == [PATH_PLAIN if short else PATH_PAIRS64], (N, T, at)
+                assert np.all(np.abs(got - whole[i:i + T]) <= 1e-13 * top[i:i + T])
