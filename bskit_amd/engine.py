@@ -589,25 +589,27 @@ class GridEngine:
         not depend on the list."""
         return int(max(8, min(1024, ncell // 256 // 8 * 8)))
 
-    def sum_path(self, fmt, tri, nfield, ncell=None):
+    def sum_path(self, fmt, tri, nfield):
         """Path of the triple sums of a list over shells of a format.
 
         FP32: the blocked path needs a plan (plan and copy 20 us) and enough
         triangles to fill the chip; both give the same bits.  Measured, us,
-        first call of a list / repeated, plain against blocked: 64^3 cells, 48
-        triangles 56/39 against 81/47; 200^3, two 72/54 against 134/111, twelve
-        153/138 against 162/132, 24 275/262 against 179/142; 256^3, twelve
-        240/225 against 243/221."""
-        ntri, ncell = len(tri), self.ncell if ncell is None else ncell
+        first call of a list / repeated on shells in the caches, plain against
+        blocked: 64^3 cells, eight triangles 53/38 against 72/46; 200^3, two
+        72/54 against 134/111, eight 114/100 against 141/115, 24 275/262 against
+        179/142; 256^3, eight 165/153 against 182/160.  In measurements of new
+        fields the two are even at eight and blocked is ahead above (twelve
+        over 128^3 226 / 220, 98 over 64^3 206 / 197 for the whole call)."""
+        ntri = len(tri)
         if fmt == L.FMT_BF16X2:
             return PATH_MFMA
         if fmt == L.FMT_F32:
-            return PATH_PLAIN if ntri <= 12 or ntri * ncell <= 3e7 else PATH_BLOCKED
-        if not self.pairs64_supported(self.nb, nfield) or self._short64(tri, nfield, ncell):
+            return PATH_PLAIN if ntri <= 8 else PATH_BLOCKED
+        if not self.pairs64_supported(self.nb, nfield) or self._short64(tri, nfield):
             return PATH_PLAIN
         return PATH_PAIRS64
 
-    def _short64(self, tri, nfield, ncell):
+    def _short64(self, tri, nfield):
         """Whether one sweep per triangle is faster than the FP64 pair kernel,
         which runs one wave per 16 pairs x 16 third sides of a workgroup's
         cells: a short list leaves the others idle.
@@ -624,7 +626,7 @@ class GridEngine:
         213, eight 335 / 321; over all of 256^3 20 586 / 1123, of 320^3 1476 /
         2732.  (On small meshes both are latencies: whole measurements with ten
         triangles over 64^3 cells 209 / 188.)"""
-        ntri = len(tri)
+        ntri, ncell = len(tri), self.ncell
         if ntri > 24:
             return False
         per = 2e-6 if ncell <= 1 << 24 else (2.4e-6 if ncell <= 1 << 25 else 3e-6)
@@ -632,7 +634,7 @@ class GridEngine:
         if sweeps > 72 + 6 * max(0.0, ncell / 65536 - 4):
             return False
         tri = np.ascontiguousarray(tri, dtype=np.int32)
-        key = (tri.tobytes(), 'short64', nfield, ncell, self.levels64())
+        key = (tri.tobytes(), 'short64', nfield, self.levels64())
         short = self._tri_cache.get(key)
         if short is None:
             part = 1.0
@@ -854,7 +856,7 @@ class GridEngine:
             L.call('bsk_shells', self._plan, dt, L.KIND_DELTA, L.ptr(dks[f]), 0, nb, 0, xs,
                    L.STAGE_X, fmt, None, None, cells, 0, L.ptr(works[f]), st)
         part = torch.empty(T, dtype=torch.float64, device=self.device)
-        sums = PATH_PLAIN if f64 else self.sum_path(fmt, tri, nf, cells)
+        sums = PATH_PLAIN if f64 else self.sum_path(fmt, tri, nf)
         if path == PATH_MFMA:
             plan = self.pair_plan(tri, nb, _MODE[nf], levels=False)
             nwg = int(nwg) if nwg else int(max(1, min(1024, cells // 128 // 8)))
