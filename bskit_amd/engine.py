@@ -922,9 +922,6 @@ class GridEngine:
         T, nb = len(tri), self.nb
         key = (np.ascontiguousarray(tri).tobytes(), 'gridinfo')
         plan = self._tri_cache.get(key)
-        if plan is None:
-            with torch.cuda.device(self.device):
-                plan = self._tri_cache[key] = PairPlan(tri, nb, L.MODE_AUTO, gridinfo=True)
         # x slabs whose shells, weights and intermediates fit max_bytes (one
         # plane at least), all in the same buffer
         slabs, x0, end = [], 0, self.S // 2 + 1
@@ -945,6 +942,12 @@ class GridEngine:
             weight, wk = buf[2 * nb * n:], buf[(2 * nb + 1) * n:]
             L.call('bsk_gridinfo_shells', self._plan, x0, x1, L.ptr(buf), n, L.ptr(weight),
                    L.ptr(wk), s)
+            if plan is None:
+                # a new list (the usual case: a binning's grid info is asked for
+                # once) is planned while the first shells are made: 8 / 16 / 32
+                # bins 240 / 507 / 2270 -> 218 / 433 / 1970 us
+                with torch.cuda.device(self.device):
+                    plan = self._tri_cache[key] = PairPlan(tri, nb, L.MODE_AUTO, gridinfo=True)
             # at least four 64-cell chunks per workgroup, at most 256 MB of
             # partials (2 KB per item and workgroup)
             nwg = int(max(8, min(512, n // 256, (1 << 17) // plan.nitem) // 8 * 8))
