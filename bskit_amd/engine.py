@@ -1003,11 +1003,12 @@ class GridEngine:
         dt = L.DT_F32 if dk.dtype == torch.complex64 else L.DT_F64
         nbytes = L.size_out()
         L.call('bsk_power_spectrum_workspace', self._plan, ctypes.byref(nbytes))
-        w = (work or self.work).get('pk', nbytes.value)
-        out = torch.empty(3 * self.nb, dtype=torch.float64, device=self.device)
-        L.call('bsk_power_spectrum', self._plan, dt, L.ptr(dk), L.ptr(out), L.ptr(w),
-               stream_handle(stream))
-        s = out.view(self.nb, 3).cpu().numpy()
+        with torch.cuda.stream(stream):  # buffers, kernels and the copy to the host
+            w = (work or self.work).get('pk', nbytes.value)
+            out = torch.empty(3 * self.nb, dtype=torch.float64, device=self.device)
+            L.call('bsk_power_spectrum', self._plan, dt, L.ptr(dk), L.ptr(out), L.ptr(w),
+                   stream_handle())
+            s = out.view(self.nb, 3).cpu().numpy()
         nmodes = s[:, 1]
         with np.errstate(divide='ignore', invalid='ignore'):
             p = np.where(nmodes > 0, self.box ** 3 * s[:, 0] / nmodes, np.nan)

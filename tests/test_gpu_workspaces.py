@@ -102,3 +102,22 @@ def test_grid_info_stream(nb):
     for (n0, k0), b in zip(want, (1 << 22, None)):
         n1, k1 = eng.grid_info(tri, max_bytes=b, stream=side)
         assert np.array_equal(n1, n0) and np.array_equal(k1, k0, equal_nan=True)
+
+
+def test_power_spectrum_stream():
+    """power_spectrum on a stream that still has work queued."""
+    eng, _, _ = setup(128, 16)
+    g = torch.Generator(device='cuda')
+    g.manual_seed(5)
+    dk = eng.forward(torch.randn((128,) * 3, generator=g, device='cuda'))
+    want = eng.power_spectrum(dk)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        x = torch.ones((4096, 4096), device='cuda')
+        for _ in range(20):
+            x = x @ x
+            x /= x.max()
+    got = eng.power_spectrum(dk, stream=side)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
