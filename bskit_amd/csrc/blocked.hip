@@ -9,9 +9,9 @@
 //
 //  * k_triple_blocked (BS = 4): the 16 waves of a workgroup run 16 tiles over
 //    the same cells from shells staged in LDS, so the shells are read from L2
-//    once per 16 tiles.  1.78 ms for the list above, bound by VALU issue
-//    (5500 multiplies and multiply-adds per cell with the tiles' unused
-//    thirds, unpacked: 1.3 ms at 2.1 GHz).  Eight waves and eight tiles per
+//    once per 16 tiles.  1.9-2.0 ms for the list above, bound by VALU issue
+//    (81% of the time; 5500 multiplies and multiply-adds per cell with the
+//    tiles' unused thirds, unpacked: 1.3 ms at 2.1 GHz).  Eight waves and eight tiles per
 //    workgroup took 2.0 ms (twice the L2 reads), waves that read their tile's
 //    shells from L2 by themselves 2.5 ms, quarter-wide tiles (BS = 2) 4.5 ms.
 //    The sums of two of a vector's four cells are formed at a time: with all
@@ -508,7 +508,7 @@ int launch_blocked(const BlockTables& t, BlockedArgs a, double scale, double* ou
 //  * else direct or blocked by their estimated times.  A workgroup of blocked
 //    takes about 125 us for a chunk of 65536 cells, one at a time on a CU;
 //    direct reads its tiles' shells from the caches at about 15 TB/s.  512^3,
-//    3624 triangles 42400 / 4660 / 1780; 256^3, 564 triangles (62 chunks) 3200 /
+//    3624 triangles 42400 / 4660 / 1950; 256^3, 564 triangles (62 chunks) 3200 /
 //    400 / 245; <ABC>, 407 triangles over 64^3 cells 63 / 43 / 120.
 // A launch of direct or blocked must hold one group at least (group_batch).
 enum Way { kPlain, kDirect, kStaged };

@@ -27,8 +27,8 @@
 //     its T^3 nodes into fixed point in LDS: of its own particles and of those
 //     classes of the seven tiles below that reach it (1.2 records per particle
 //     in all), then writes its nodes as float.
-// 256^3 particles on 512^3: 0.53 ms (bin 161 us, place 144, tile 219: the LDS
-// atomics; 0.8 GB cross HBM at least).  Tiles that summed only their own
+// 256^3 particles on 512^3: 0.53 ms (bin 161 us, bound by VALU issue; place
+// 159, by memory; tile 221, by VALU issue and the LDS atomics).  Tiles that summed only their own
 // particles, wrote the shared face nodes to a boundary record of 400 MB and left
 // them to a pass of its own took 375 + 329 us for the tile step.
 // Other N (and 2^29 or more particles on one tile): fixed-point 64-bit atomics
@@ -102,7 +102,8 @@ constexpr int kPU = 4;  // particles per thread of k_cic_bin (169 us with one, 1
 // (neighbouring particles of a catalogue usually share bins) get consecutive
 // slots from a single atomic add of their count.  The groups are found first,
 // then all groups' atomics are in flight together (one at a time, each waiting
-// for the last, took 372 us for 256^3 particles; this 155, bound by the atomics).
+// for the last, took 372 us for 256^3 particles; this 155-161, VALU issue 84% of
+// the time: the search for the groups).
 __global__ __launch_bounds__(256) void k_cic_bin(const float* __restrict__ pos, long long np, int N,
                                                  float to_mesh, uint32_t* __restrict__ count,
                                                  uint32_t* __restrict__ slot) {

@@ -5,15 +5,16 @@
 // of 16 third-side shells, launch segments over the sublattice levels), the
 // arithmetic all FP64: a K step of eight cells is, per item, two
 // v_mfma_f64_16x16x4 on the pair products (A) and the shells (B).  One item
-// costs 512 multiply-adds per cell whatever its tile needs of them, but its
+// costs 256 multiply-adds per cell whatever its tile needs of them, but its
 // 16 x 16 accumulators are 8 VGPRs a lane, so eight waves hold every item of
 // a segment and the shells are read once; a register-blocked sum of single
 // triangles (blocked.hip's scheme in FP64) holds 64 triangles a wave and read
 // the shells 13 times: 5.0 ms at 512^3 / 32 bins, one sweep per triangle 84 ms,
-// this 0.90 ms over the levels (1.95 without them).  FP64 MFMA and FP64 VALU
+// this 0.96 ms over the levels (2.0 without them).  FP64 MFMA and FP64 VALU
 // have the same peak on gfx950 (72 TFLOP/s measured with a large matrix
 // product) and share issue time, so what bounds it is the MFMAs (0.55 ms of
-// the 0.90 at 2.17 GHz), every VALU instruction between them (the K loop is
+// the 0.96 at 2.17 GHz; matrix cores 68% busy in the segments of many items,
+// 41% in the thin ones), every VALU instruction between them (the K loop is
 // rolled with one address add per LDS read) and, in the thin segments, the
 // latency of one wave's K steps.
 //

@@ -1,14 +1,17 @@
 // Triple-product reductions sum_x A_i(x) B_j(x) C_k(x) over the N^3 cells.
 //
-// Three device paths:
+// Two of the device paths:
 //  * plain : one sweep over the cells per triangle, reading three shells,
 //            FP32 (or FP64) products and per-thread accumulation, FP64
 //            workgroup sums -- the structure of the reference's
-//            np.sum(d_i*d_j*d_k) loop.
+//            np.sum(d_i*d_j*d_k) loop.  For lists of a few triangles, for
+//            more shells than the others hold and for FP64 x slabs.
 //  * tiled : cells staged through LDS in chunks, each thread owns a few
-//            triangles; used in FP64 for the grid-info sums (N_tri and the
-//            three k-mean numerators share their pair products).
-//  * mfma  : split-BF16 MFMA GEMMs, in mfma.hip.
+//            triangles; in FP64 for the grid-info sums of more than 136 bins
+//            (N_tri and the three k-mean numerators share their pair products).
+// The others: blocked.hip (FP32, blocks of triangles per sweep, the bits of
+// plain), dpairs.hip (FP64 MFMA over pair lists, also weighted for grid info),
+// mfma.hip (split-BF16 MFMA over pair lists).
 // All paths write per-workgroup partials that a second kernel reduces in a
 // fixed order in FP64, so a result does not depend on what else runs.
 #include "launch.h"
