@@ -19,7 +19,16 @@
 //   G[kind][b][x][ny][nz]   after x, each sum stored at (ny, nz) and (nz, ny):
 //                           the y step reads rows (245 us with one copy, 145)
 //   H[kind][b][row][nz]     after y, row = x (x + 1) / 2 + y
-//   shells [kind][b][cell]  cell = x (x + 1) (x + 2) / 6 + y (y + 1) / 2 + z
+//   shells [kind][b][place]  place = cells - 1 - cell,
+//                           cell = x (x + 1) (x + 2) / 6 + y (y + 1) / 2 + z
+//
+// The cells go from the corner of the wedge to the origin.  A shell field is as
+// large at the origin as its mode count and falls off from there, so the sums add
+// small products first; the origin's, 10^3 times the others' and more, is the
+// last of the last workgroup, whose partial the reduction adds last.  Summed from
+// the origin outwards every cell is rounded at the size of that product: counts
+// of 1e13 to 3e13 (768^3 mesh, bins of 33 k_f) were 0.136 off a whole number
+// (rms), now 0.006, with the tiled sums over every cell 0.038.
 #include "launch.h"
 
 namespace {
@@ -52,12 +61,12 @@ __global__ __launch_bounds__(64) void k_gi_weights(GridInfoArgs a) {
     return;
   }
   if (y > x) return;
-  const long long base = tri3(x) - tri3(a.x0) + tri2(y);
+  const long long place = a.cells - 1 - (tri3(x) - tri3(a.x0) + tri2(y));
   for (int z = threadIdx.x; z <= y; z += 64) {
     const int sign = ((x == 0 || x == h) ? 1 : 2) * ((y == 0 || y == h) ? 1 : 2) *
                      ((z == 0 || z == h) ? 1 : 2);
     const int perm = (x == y && y == z) ? 1 : ((x == y || y == z) ? 3 : 6);
-    a.weight[base + z] = (double)(sign * perm);
+    a.weight[place - z] = (double)(sign * perm);
   }
 }
 
@@ -173,7 +182,7 @@ __global__ __launch_bounds__(256) void k_gi_z(const double* __restrict__ cn,
     hu[j] = h + ((long long)b * rows + r) * a.NP;
     hk[j] = hu[j] + a.nb * rows * a.NP;
   }
-  const long long cell0 = tri3(x) - tri3(a.x0);
+  const long long place0 = a.cells - 1 - (tri3(x) - tri3(a.x0));
   for (int z0 = 0; z0 <= y0 + nrow - 1; z0 += 64) {
     const int z = z0 + lane, zc = z < a.XP ? z : a.XP - 1;
     double u[kZT], k[kZT];
@@ -195,7 +204,7 @@ __global__ __launch_bounds__(256) void k_gi_z(const double* __restrict__ cn,
     for (int j = 0; j < kZT; ++j) {
       const int y = y0 + j;
       if (j < nrow && z <= y) {
-        const long long o = (long long)b * a.stride + cell0 + tri2(y) + z;
+        const long long o = (long long)b * a.stride + place0 - tri2(y) - z;
         f[o] = u[j];
         f[a.nb * a.stride + o] = k[j];
       }

@@ -938,7 +938,9 @@ class GridEngine:
         s = stream_handle()
         buf = torch.empty(max(v[3] for v in slabs) // 8, dtype=torch.float64, device=self.device)
         total = None
-        for x0, x1, n, _ in slabs:  # shells, weights and intermediates
+        # shells, weights and intermediates, from the far slab to the origin's
+        # (small sums first)
+        for x0, x1, n, _ in reversed(slabs):
             weight, wk = buf[2 * nb * n:], buf[(2 * nb + 1) * n:]
             L.call('bsk_gridinfo_shells', self._plan, x0, x1, L.ptr(buf), n, L.ptr(weight),
                    L.ptr(wk), s)

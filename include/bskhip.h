@@ -366,8 +366,9 @@ int bsk_triples_f64(const bsk_pairs* pairs, const double* f_i, const double* f_j
  * is the sum over the cells S/2 >= x >= y >= z >= 0 weighted by the orbits'
  * sizes.  bsk_gridinfo_shells makes the FP64 unit shells (rows 0..nbin-1) and
  * |k| shells (rows nbin..2 nbin-1) of the wedge planes [x0, x1) and the
- * weights; bsk_gridinfo_layout gives the cells of a row (padded to 64, the
- * padding weighted 0) and the workspace.  bsk_gridinfo_pairs plans the four
+ * weights, in descending order of (x, y, z): the sums take the origin's product,
+ * by far the largest, last; bsk_gridinfo_layout gives the cells of a row (padded
+ * to 64, the padding weighted 0) and the workspace.  bsk_gridinfo_pairs plans the four
  * sums of each triangle (i, j, k) for bsk_triples_f64 (out[4t]: n_i n_j n_k,
  * out[4t + 1 + e]: side e's unit shell replaced by its |k| shell).  Replaces
  * measure_gridinfo_faster's shells and sums (bskit/main.py:2006-2064). */
