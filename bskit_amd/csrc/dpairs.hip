@@ -47,6 +47,15 @@ constexpr int kCK = kDPairChunk;      // cells per staged chunk
 constexpr int kLD = kCK + 4;          // LDS row stride (doubles)
 constexpr int kSEG = kCK / 2;         // 16-byte segments per row
 constexpr int kSteps = kCK / 8;       // K steps of eight cells per chunk
+// Chunks added in one chain, whose sum then goes to a second accumulator: a
+// chain over all of a workgroup's cells (8000 at 200^3, 55000 at 384^3) is
+// rounded at its full size every time.  Error over sqrt(sum of term^2) in C
+// order, one chain / this / one sweep per triangle: 200^3 8.9e-15 / 2.5e-15 /
+// 0.9e-15, 384^3 2.0e-14 / 1.7e-15 / 1.0e-15; over the levels, where the shells'
+// own rounding shows, 4.4e-15 / 3.1e-15 and 8.9e-15 / 2.9e-15.  At the same speed
+// (<AAB> of 100 shells 2% slower).  The weighted sums (grid info) run in one
+// chain: their cells come in ascending order of size.
+constexpr int kRun = 8;
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double d2 __attribute__((ext_vector_type(2)));
@@ -80,7 +89,7 @@ BSK_DEV void run_items(const DPairArgs& a, double* smem, const int* items, const
   // read row 0: their sums are never read) and of its third-side row
   constexpr int NC = CNT ? CNT : 1;
   int desc[NC], oi[NC], oj[NC], ok[NC];
-  d4 acc[NC];
+  d4 acc[NC], sum[NC];
 #pragma unroll
   for (int s = 0; s < CNT; ++s) {
     desc[s] = __builtin_amdgcn_readfirstlane(items[s]);
@@ -90,7 +99,7 @@ BSK_DEV void run_items(const DPairArgs& a, double* smem, const int* items, const
     oi[s] = (s0 + ia) * kLD + 2 * grp;
     oj[s] = ((SETS == 3 ? s1 : s0) + ib) * kLD + 2 * grp;
     ok[s] = (R.r2 + 16 * ((desc[s] >> 16) & 0xff) + col) * kLD + 2 * grp;
-    acc[s] = d4{0.0, 0.0, 0.0, 0.0};
+    acc[s] = sum[s] = d4{0.0, 0.0, 0.0, 0.0};
   }
 
   // staging: segment v = thread + k kNT is 16 bytes of staged row v / kSEG:
@@ -98,53 +107,75 @@ BSK_DEV void run_items(const DPairArgs& a, double* smem, const int* items, const
   const int n = a.nsh, nrow = SETS * n + (WT ? 1 : 0);
   const int nch = (int)(a.ncell / kCK);
   const int ch0 = (int)((long long)nch * lw / a.nwg), ch1 = (int)((long long)nch * (lw + 1) / a.nwg);
-  const double* src[PV];
-  int dst[PV];
+  // One set of many shells: a thread's rows are kRows apart, and one pointer does
+  // for all of them (the registers would spill: 154 against 162 ms for 272 shells
+  // of 192^3); the address additions cost fewer shells 2%
+  constexpr bool kOne = SETS == 1 && !WT && PV > 10;
+  constexpr int kRows = kNT / kSEG, KP = kOne ? 1 : PV;
+  const int row0 = threadIdx.x / kSEG, sg0 = threadIdx.x % kSEG;
+  const double* src[KP];
+  int dst[KP];
 #pragma unroll
-  for (int k = 0; k < PV; ++k) {
-    const int v = threadIdx.x + k * kNT, row = v / kSEG, sg = v % kSEG;
+  for (int k = 0; k < KP; ++k) {
+    const int row = row0 + k * kRows;
     const int set = row < n ? 0 : (row < 2 * n ? 1 : 2);  // the set's place in the list
     const int sh = row - set * n;
     const bool wt = WT && row == nrow - 1;
-    const double* base = set == 0 ? a.f[0] : (SETS == 3 && set == 1 ? a.f[1] : a.f[2]);
+    const double* base = kOne || set == 0 ? a.f[0] : (SETS == 3 && set == 1 ? a.f[1] : a.f[2]);
     const int lrow = set == 0 ? s0 : (SETS == 3 && set == 1 ? s1 : s2);
-    src[k] = (wt ? a.weight : base + sh * a.stride) + 2 * sg + (long long)ch0 * kCK;
-    dst[k] = row < nrow ? (wt ? R.rw : lrow + sh) * kLD + 2 * sg : -1;
+    src[k] = (wt ? a.weight : base + (kOne ? row : sh) * a.stride) + 2 * sg0 + (long long)ch0 * kCK;
+    dst[k] = kOne || row < nrow ? (wt ? R.rw : (kOne ? s0 + row : lrow + sh)) * kLD + 2 * sg0 : -1;
   }
+  auto staged = [&](int k) { return kOne ? row0 + k * kRows < n : dst[k] >= 0; };
   d2 pre[PV];
   auto fetch = [&]() {
 #pragma unroll
-    for (int k = 0; k < PV; ++k) {
-      if (dst[k] >= 0) pre[k] = *reinterpret_cast<const d2*>(src[k]);
-      src[k] += kCK;
-    }
+    for (int k = 0; k < PV; ++k)
+      if (staged(k))
+        pre[k] = *reinterpret_cast<const d2*>(kOne ? src[0] + (long long)(k * kRows) * a.stride : src[k]);
+#pragma unroll
+    for (int k = 0; k < KP; ++k) src[k] += kCK;
   };
-  if (ch0 < ch1) fetch();
-  for (int ch = ch0; ch < ch1; ++ch) {
-    __syncthreads();  // every wave is done with the previous chunk
+  auto put = [&]() {
 #pragma unroll
     for (int k = 0; k < PV; ++k)
-      if (dst[k] >= 0) *reinterpret_cast<d2*>(smem + dst[k]) = pre[k];
-    __syncthreads();
-    if (ch + 1 < ch1) fetch();  // the next chunk's loads overlap this one's math
-    if (CNT == 0) continue;
+      if (staged(k))
+        *reinterpret_cast<d2*>(smem + (kOne ? dst[0] + k * kRows * kLD : dst[k])) = pre[k];
+  };
+  if (ch0 < ch1) fetch();
+  for (int ch = ch0; ch < ch1;) {
+    const int end = WT || ch1 - ch <= kRun ? ch1 : ch + kRun;
+    for (; ch < end; ++ch) {
+      __syncthreads();  // every wave is done with the previous chunk
+      put();
+      __syncthreads();
+      if (ch + 1 < ch1) fetch();  // the next chunk's loads overlap this one's math
+      if (CNT == 0) continue;
 #pragma unroll 1
-    for (int ks = 0; ks < kSteps; ++ks) {
-      int o = 8 * ks;
-      asm("" : "+s"(o));  // keeps one add per read, not an induction variable per row
-      const double* f = smem + o;
-      d2 p = {0.0, 0.0};
+      for (int ks = 0; ks < kSteps; ++ks) {
+        int o = 8 * ks;
+        asm("" : "+s"(o));  // keeps one add per read, not an induction variable per row
+        const double* f = smem + o;
+        d2 p = {0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < CNT; ++s) {
+          const d2 z = *reinterpret_cast<const d2*>(f + ok[s]);
+          if (s == 0 || desc[s] < 0) {  // uniform: new tile, new pair products
+            const d2 x = *reinterpret_cast<const d2*>(f + oi[s]);
+            const d2 y = *reinterpret_cast<const d2*>(f + oj[s]);
+            p = x * y;
+            if (WT) p *= *reinterpret_cast<const d2*>(f + R.rw * kLD + 2 * grp);
+          }
+          acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(p.x, z.x, acc[s], 0, 0, 0);
+          acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(p.y, z.y, acc[s], 0, 0, 0);
+        }
+      }
+    }
+    if constexpr (!WT) {
 #pragma unroll
       for (int s = 0; s < CNT; ++s) {
-        const d2 z = *reinterpret_cast<const d2*>(f + ok[s]);
-        if (s == 0 || desc[s] < 0) {  // uniform: new tile, new pair products
-          const d2 x = *reinterpret_cast<const d2*>(f + oi[s]);
-          const d2 y = *reinterpret_cast<const d2*>(f + oj[s]);
-          p = x * y;
-          if (WT) p *= *reinterpret_cast<const d2*>(f + R.rw * kLD + 2 * grp);
-        }
-        acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(p.x, z.x, acc[s], 0, 0, 0);
-        acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(p.y, z.y, acc[s], 0, 0, 0);
+        sum[s] += acc[s];
+        acc[s] = d4{0.0, 0.0, 0.0, 0.0};
       }
     }
   }
@@ -154,7 +185,7 @@ BSK_DEV void run_items(const DPairArgs& a, double* smem, const int* items, const
   for (int s = 0; s < CNT; ++s) {
     const int pos = __builtin_amdgcn_readfirstlane(outpos[s]) - a.item0;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) out[(long long)pos * 256 + (4 * r + grp) * 16 + col] = acc[s][r];
+    for (int r = 0; r < 4; ++r) out[(long long)pos * 256 + (4 * r + grp) * 16 + col] = (WT ? acc : sum)[s][r];
   }
 }
 
@@ -167,8 +198,16 @@ BSK_DEV void run_count(int cnt, const DPairArgs& a, double* smem, const int* ite
     run_count<CNT - 1, PV, SETS, WT>(cnt, a, smem, items, outpos, lw);
 }
 
+// Waves per SIMD that the registers must allow: eight (four workgroups per CU)
+// for the thin segments, as the mesh gives 1024 at most and three would leave a
+// quarter of them for a second round (4% slower); four or two above.
+constexpr int waves(int ni, int pv, bool wt) {
+  if (wt) return ni <= 4 && pv <= 10 ? 4 : 2;
+  return ni * pv <= 6 ? 8 : (ni * pv <= 20 ? 4 : 2);
+}
+
 template <int NI, int PV, int SETS, bool WT>
-__global__ __launch_bounds__(kNT, NI <= 4 && PV <= 10 ? 4 : 2) void k_triple_dpairs(DPairArgs a) {
+__global__ __launch_bounds__(kNT, waves(NI, PV, WT)) void k_triple_dpairs(DPairArgs a) {
   extern __shared__ __attribute__((aligned(16))) double smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int lw = blockIdx.x, pass = 0;  // cell range and item-list pass (see PairArgs)
