@@ -201,19 +201,29 @@ class PairPlan:
             L.call('bsk_pairs_create_levels', ctypes.byref(h), int(mode), int(nshell), len(tri),
                    tri.ctypes.data_as(ip), levels.ctypes.data_as(ip))
         self.handle = h
-        ns = ctypes.c_int()
-        arr = [(ctypes.c_int * 4)() for _ in range(6)]
-        L.call('bsk_pairs_segments', h, ctypes.byref(ns), *arr)
-        # launch segments: (layout parts bitmask, first shell, shells staged,
-        # launches, items per wave, replicas of the wave lists)
-        self.segments = [tuple(a[g] for a in arr) for g in range(ns.value)]
-        self.list_entries = sum(8 * g[3] * g[4] for g in self.segments)
+        self._segments = None
         if upload:
             L.call('bsk_pairs_upload', h)
         self.ntri = len(tri)
         v = [ctypes.c_int() for _ in range(5)]
         L.call('bsk_pairs_info', h, *[ctypes.byref(x) for x in v])
         self.npair, self.ntile, self.nitem, self.items_per_wave, self.npass = [x.value for x in v]
+
+    @property
+    def segments(self):
+        """Launch segments: (layout parts bitmask, first shell, shells staged,
+        launches, items per wave, replicas of the wave lists).  Read when asked
+        for: measurements plan a list without it."""
+        if self._segments is None:
+            ns = ctypes.c_int()
+            arr = [(ctypes.c_int * 4)() for _ in range(6)]
+            L.call('bsk_pairs_segments', self.handle, ctypes.byref(ns), *arr)
+            self._segments = [tuple(a[g] for a in arr) for g in range(ns.value)]
+        return self._segments
+
+    @property
+    def list_entries(self):
+        return sum(8 * g[3] * g[4] for g in self.segments)
 
     def tables(self):
         """(items, partial positions, pair rows) host tables of the launches."""
