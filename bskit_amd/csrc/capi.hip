@@ -866,22 +866,43 @@ struct PairTiles {
 
 long long pkey(int a, int b) { return ((long long)a << 32) | (unsigned)b; }
 
+// Shells n of a table of all n^2 pairs, where it is no larger than a sort of the
+// list's own would be (a list of 3624 triangles is planned in a third of the
+// time, one of 49781 in a quarter); 0: sort.
+size_t table_side(int top, size_t entries) {
+  const size_t n = (size_t)top + 1;
+  return n * n <= 4 * entries + 4096 ? n : 0;
+}
+
+size_t dense_pairs(const std::vector<Role>& roles) {
+  int top = 0;
+  for (const Role& r : roles) top = std::max(top, std::max(r.a, r.b));
+  return table_side(top, roles.size());
+}
+
 // Distinct pairs sorted by the set of third-side blocks they need (then by
 // (a, b)) and packed into 16-row tiles in that order; a tile's items are the
 // union of its rows' blocks.  exact: a new tile at every change of the block
 // set (no MFMA on a block a row does not need); otherwise every tile is
 // filled (fewer tiles, so fewer pair products and pair-side LDS reads).
 PairTiles build_tiles(const std::vector<Role>& roles, bool exact) {
-  std::vector<std::pair<long long, unsigned>> pm;
-  pm.reserve(roles.size());
-  for (const Role& r : roles) pm.push_back({pkey(r.a, r.b), 1u << (r.c / 16)});
-  std::sort(pm.begin(), pm.end());
   std::vector<std::pair<long long, unsigned>> uniq;
-  for (const auto& e : pm) {
-    if (!uniq.empty() && uniq.back().first == e.first)
-      uniq.back().second |= e.second;
-    else
-      uniq.push_back(e);
+  if (const size_t n = dense_pairs(roles)) {
+    std::vector<unsigned> mask(n * n, 0u);
+    for (const Role& r : roles) mask[r.a * n + r.b] |= 1u << (r.c / 16);
+    for (size_t k = 0; k < n * n; ++k)
+      if (mask[k]) uniq.push_back({pkey((int)(k / n), (int)(k % n)), mask[k]});
+  } else {
+    std::vector<std::pair<long long, unsigned>> pm;
+    pm.reserve(roles.size());
+    for (const Role& r : roles) pm.push_back({pkey(r.a, r.b), 1u << (r.c / 16)});
+    std::sort(pm.begin(), pm.end());
+    for (const auto& e : pm) {
+      if (!uniq.empty() && uniq.back().first == e.first)
+        uniq.back().second |= e.second;
+      else
+        uniq.push_back(e);
+    }
   }
   std::stable_sort(uniq.begin(), uniq.end(),
                    [](const std::pair<long long, unsigned>& x,
@@ -939,30 +960,62 @@ std::vector<Role> assign_roles(int mode, int option, int ntri, const int* tri) {
 std::vector<Role> assign_roles_cover(int ntri, const int* tri) {
   std::vector<std::array<Role, 3>> cand(ntri);
   std::vector<int> ncand(ntri, 0);
-  std::vector<std::pair<long long, int>> pt;  // (pair key, triangle)
-  pt.reserve((size_t)3 * ntri);
+  int top = 0;
+  size_t ncands = 0;
   for (int t = 0; t < ntri; ++t) {
     int v[3] = {tri[3 * t], tri[3 * t + 1], tri[3 * t + 2]};
     std::sort(v, v + 3);
+    top = std::max(top, v[2]);
     const Role opts[3] = {{v[2], v[1], v[0]}, {v[1], v[0], v[2]}, {v[2], v[0], v[1]}};
     for (const Role& o : opts) {
       bool dup = false;
       for (int q = 0; q < ncand[t]; ++q)
         dup |= cand[t][q].a == o.a && cand[t][q].b == o.b && cand[t][q].c == o.c;
-      if (dup) continue;
-      cand[t][ncand[t]++] = o;
-      pt.push_back({pkey(o.a, o.b), t});
+      if (!dup) cand[t][ncand[t]++] = o;
     }
+    ncands += ncand[t];
   }
-  std::sort(pt.begin(), pt.end());
+  // the pairs in ascending order, triangles of key i: pt[start[i] .. start[i+1])
   std::vector<long long> keys;
-  std::vector<size_t> start;  // triangles of key i: pt[start[i] .. start[i+1])
-  for (size_t e = 0; e < pt.size(); ++e)
-    if (e == 0 || pt[e].first != pt[e - 1].first) {
-      keys.push_back(pt[e].first);
-      start.push_back(e);
+  std::vector<size_t> start;
+  std::vector<int> pt(ncands);
+  const size_t n = table_side(top, ncands);
+  std::vector<int> at(n * n, 0);  // table: count of a pair, then its key, -1 for none
+  if (n) {
+    for (int t = 0; t < ntri; ++t)
+      for (int q = 0; q < ncand[t]; ++q) ++at[cand[t][q].a * n + cand[t][q].b];
+    size_t sum = 0;
+    for (size_t k = 0; k < n * n; ++k) {
+      const int c = at[k];
+      at[k] = c ? (int)keys.size() : -1;
+      if (!c) continue;
+      keys.push_back(pkey((int)(k / n), (int)(k % n)));
+      start.push_back(sum);
+      sum += c;
     }
-  start.push_back(pt.size());
+    start.push_back(sum);
+    std::vector<size_t> end(start.begin(), start.end() - 1);
+    for (int t = 0; t < ntri; ++t)
+      for (int q = 0; q < ncand[t]; ++q) pt[end[at[cand[t][q].a * n + cand[t][q].b]]++] = t;
+  } else {
+    std::vector<std::pair<long long, int>> e;  // (pair key, triangle)
+    e.reserve(ncands);
+    for (int t = 0; t < ntri; ++t)
+      for (int q = 0; q < ncand[t]; ++q) e.push_back({pkey(cand[t][q].a, cand[t][q].b), t});
+    std::sort(e.begin(), e.end());
+    for (size_t i = 0; i < e.size(); ++i) {
+      if (i == 0 || e[i].first != e[i - 1].first) {
+        keys.push_back(e[i].first);
+        start.push_back(i);
+      }
+      pt[i] = e[i].second;
+    }
+    start.push_back(e.size());
+  }
+  auto index = [&](const Role& r) -> size_t {
+    if (n) return (size_t)at[r.a * n + r.b];
+    return (size_t)(std::lower_bound(keys.begin(), keys.end(), pkey(r.a, r.b)) - keys.begin());
+  };
   std::vector<char> covered(ntri, 0);
   std::vector<int> rank(keys.size(), -1);
   std::priority_queue<std::pair<int, long long>> heap;  // (count, -key index)
@@ -974,21 +1027,20 @@ std::vector<Role> assign_roles_cover(int ntri, const int* tri) {
     heap.pop();
     const size_t i = (size_t)(-top.second);
     int cnt = 0;
-    for (size_t e = start[i]; e < start[i + 1]; ++e) cnt += !covered[pt[e].second];
+    for (size_t e = start[i]; e < start[i + 1]; ++e) cnt += !covered[pt[e]];
     if (cnt == 0) continue;
     if (cnt < top.first) {
       heap.push({cnt, top.second});
       continue;
     }
     rank[i] = nrank++;
-    for (size_t e = start[i]; e < start[i + 1]; ++e) covered[pt[e].second] = 1;
+    for (size_t e = start[i]; e < start[i + 1]; ++e) covered[pt[e]] = 1;
   }
   std::vector<Role> r(ntri);
   for (int t = 0; t < ntri; ++t) {
     int best = -1, br = INT_MAX;
     for (int q = 0; q < ncand[t]; ++q) {
-      const long long k = pkey(cand[t][q].a, cand[t][q].b);
-      const size_t i = (size_t)(std::lower_bound(keys.begin(), keys.end(), k) - keys.begin());
+      const size_t i = index(cand[t][q]);
       if (rank[i] >= 0 && rank[i] < br) {
         br = rank[i];
         best = q;
@@ -1032,6 +1084,7 @@ LevelPlan plan_level(int mode, int nkb, int cap, const std::vector<int>& idx, co
   const int nopt = given ? 0 : (mode == BSK_MODE_AUTO && !f64 ? 4 : 1);
   bool first = true;
   if (given) {
+    lp.roles.reserve(idx.size());
     for (int t : idx) lp.roles.push_back((*given)[t]);
     lp.tiles = build_tiles(lp.roles, false);
   }
@@ -1331,17 +1384,24 @@ int make_pairs(bsk_pairs** out, int mode, int nshell, int ntri, const int* tri, 
       }
     }
     // slot: item * 256 + row * 16 + column, the triangle's level in bits 28-29
-    std::vector<long long> keys(tl.pairs.size());
-    for (size_t p = 0; p < keys.size(); ++p) keys[p] = tl.pairs[p].first;
-    std::vector<size_t> kidx(keys.size());
-    for (size_t p = 0; p < kidx.size(); ++p) kidx[p] = p;
-    std::sort(kidx.begin(), kidx.end(), [&](size_t x, size_t y) { return keys[x] < keys[y]; });
+    const size_t n = dense_pairs(lp[g].roles);
+    std::vector<int> at(n * n);          // table: position of a pair
+    std::vector<size_t> kidx;            // else the pairs in ascending order
+    for (size_t p = 0; p < tl.pairs.size(); ++p) {
+      const long long k = tl.pairs[p].first;
+      if (n)
+        at[(size_t)(k >> 32) * n + (size_t)(k & 0xffffffff)] = (int)p;
+      else
+        kidx.push_back(p);
+    }
+    std::sort(kidx.begin(), kidx.end(),
+              [&](size_t x, size_t y) { return tl.pairs[x].first < tl.pairs[y].first; });
     for (size_t t = 0; t < lp[g].tri.size(); ++t) {
       const Role& r = lp[g].roles[t];
-      const long long k = pkey(r.a, r.b);
-      auto it = std::lower_bound(kidx.begin(), kidx.end(), k,
-                                 [&](size_t x, long long v) { return keys[x] < v; });
-      const int p = (int)*it;
+      const int p =
+          n ? at[r.a * n + r.b]
+            : (int)*std::lower_bound(kidx.begin(), kidx.end(), pkey(r.a, r.b),
+                                     [&](size_t x, long long v) { return tl.pairs[x].first < v; });
       const int ti = where[p].first, row = where[p].second, c = r.c;
       const int it_ = item_of[(size_t)ti * nkb + c / 16];
       const int gt = lp[g].tri[t];
