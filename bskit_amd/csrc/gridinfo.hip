@@ -13,7 +13,7 @@
 // shells of both kinds 0.34 ms (x 41, y 145, z 145 us) against 2.3 ms for two
 // sets of FP64 inverse transforms, and the sums' 0.25 ms (dpairs.hip) against
 // 24 ms for every cell with a thread per triangle: a binning's grid info in
-// 0.72 ms instead of 25.5 once its list is planned, 1.97 the first time.  The y
+// 0.72 ms instead of 25.5 once its list is planned, 0.94 the first time.  The y
 // and z steps wait for their loads (VALU issue 25 and 21% of the time).
 // Intermediates, per x plane of the slab:
 //   G[kind][b][x][ny][nz]   after x, each sum stored at (ny, nz) and (nz, ny):

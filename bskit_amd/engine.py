@@ -957,7 +957,8 @@ class GridEngine:
             if plan is None:
                 # a new list (the usual case: a binning's grid info is asked for
                 # once) is planned while the first shells are made: 8 / 16 / 32
-                # bins 240 / 507 / 2270 -> 218 / 433 / 1970 us
+                # bins 240 / 507 / 2270 -> 218 / 433 / 1970 us when plans took three
+                # times as long, now 213 / 333 / 940
                 with torch.cuda.device(self.device):
                     plan = self._tri_cache[key] = PairPlan(tri, nb, L.MODE_AUTO, gridinfo=True)
             # at least four 64-cell chunks per workgroup, at most 256 MB of
