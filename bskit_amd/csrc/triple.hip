@@ -8,7 +8,8 @@
 //            more shells than the others hold and for FP64 x slabs.
 //  * tiled : cells staged through LDS in chunks, each thread owns a few
 //            triangles; in FP64 for the grid-info sums of more than 136 bins
-//            (N_tri and the three k-mean numerators share their pair products).
+//            and of long lists on the smallest meshes (N_tri and the three
+//            k-mean numerators share their pair products).
 // The others: blocked.hip (FP32, blocks of triangles per sweep, the bits of
 // plain), dpairs.hip (FP64 MFMA over pair lists, also weighted for grid info),
 // mfma.hip (split-BF16 MFMA over pair lists).

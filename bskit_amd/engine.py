@@ -898,7 +898,7 @@ class GridEngine:
         S^3 / N_tri (NaN where N_tri == 0) over FP64 unit and |k| shells, whose
         products are summed over the mesh's symmetry wedge with orbit weights
         (bsk_gridinfo_shells), in x slabs of at most max_bytes (default half of
-        free HBM)."""
+        free HBM); over the whole mesh where gridinfo_path says so."""
         tri = np.asarray(tri, dtype=np.int32).reshape(-1, 3)
         T = len(tri)
         if T == 0:
@@ -911,7 +911,7 @@ class GridEngine:
         # kernels, buffers, additions and the copy to the host all on one
         # stream: the copy waits for them, and the buffers return to its pool
         with torch.cuda.stream(stream):
-            if self.pairs64_supported(2 * self.nb, 1):
+            if self.gridinfo_path(T) == 'wedge':
                 total = self._gridinfo_wedge(tri, max_bytes)
             else:
                 total = self._gridinfo_tiled(tri, max_bytes)
@@ -921,6 +921,19 @@ class GridEngine:
         nz = ntri != 0
         kbar[nz] = sums[nz, 1:4] / ntri[nz, None]
         return ntri, kbar
+
+    def gridinfo_path(self, ntri):
+        """'wedge', or 'tiled' (whole mesh, a thread per triangle): for more
+        shells than the pair kernel holds, and for long lists on the smallest
+        meshes, where planning the list for the wedge's sums costs the host more
+        than the mesh's cells cost the GPU.  First call of a list, us, wedge /
+        tiled: 300 triangles over 16^3 cells 158-350 / 103-122, over 40^3 181-367
+        / 145-223, 3000 there 780-1028 / 368-496, 1000 over 64^3 303-844 /
+        369-927.  Repeated, the wedge's sums take 85-112, 134-149 and 120-179 us:
+        below 300 triangles and above 40^3 cells they gain as much there as the
+        plan costs."""
+        few = self.ncell > 40 ** 3 or ntri < 300
+        return 'wedge' if few and self.pairs64_supported(2 * self.nb, 1) else 'tiled'
 
     def _gridinfo_slab(self, x0, x1):
         n, nbytes = ctypes.c_longlong(), L.size_out()
@@ -975,7 +988,7 @@ class GridEngine:
 
     def _gridinfo_tiled(self, tri, max_bytes, stream=None):
         """The same sums x slab by x slab of the whole mesh with the tiled FP64
-        kernel, for more shells than the pair kernel holds."""
+        kernel (gridinfo_path)."""
         T = len(tri)
         N, nb = self.S, self.nb
         plane = N * N * 8 * 2 * nb
