@@ -736,11 +736,11 @@ class GridEngine:
             nbytes = L.size_out()
             L.call('bsk_triples_plain_workspace', min(T, 65535), nchunk, ctypes.byref(nbytes))
             w = (work or self.work).get('plain', nbytes.value)
+            pt, po = tri_d.data_ptr(), out.data_ptr()  # (views cost short lists 5 us)
             for t0 in range(0, T, 65535):
-                t1 = min(T, t0 + 65535)
                 L.call('bsk_triples_plain', dt, L.ptr(sa.data), L.ptr(sb.data), L.ptr(sc.data),
-                       sa.stride, sa.sum_cells, t1 - t0, L.ptr(tri_d[t0:t1]), nchunk, float(scale),
-                       L.ptr(out[t0:t1]), L.ptr(w), s)
+                       sa.stride, sa.sum_cells, min(T - t0, 65535), ctypes.c_void_p(pt + 12 * t0),
+                       nchunk, float(scale), ctypes.c_void_p(po + 8 * t0), L.ptr(w), s)
             return out
         if path == PATH_BLOCKED:
             if any(x.fmt != L.FMT_F32 for x in sets):
