@@ -2,7 +2,7 @@
 
 Nothing in the product (``bskit_amd``) imports, links or runs anything from
 this package.  Only ``tests/``, ``__graft_entry__.smoke()`` and the
-``cpu_baseline`` leg of ``bench.py`` use it, and only as the checker.
+``cpu_baseline`` leg of ``bench.py`` use it, and only to compare with.
 
 Contents
 --------
